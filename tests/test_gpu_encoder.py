@@ -114,6 +114,41 @@ def test_encoder_parity_narrow_ragged(device, cfg):
 
 @pytest.mark.parametrize(
     "cfg",
+    [TransformerConfig(3, 1, 32, 1, 64, 2, True), TransformerConfig(9, 16, 64, 2, 32, 2, False),
+     TransformerConfig(5, 17, 64, 1, 128, 2, True), TransformerConfig(33, 32, 32, 4, 128, 2, False),
+     TransformerConfig(80, 33, 64, 8, 64, 2, True), TransformerConfig(16, 97, 128, 2, 128, 2, True),
+     TransformerConfig(17, 127, 128, 1, 32, 2, False), TransformerConfig(65, 112, 128, 4, 64, 2, True),
+     TransformerConfig(160, 128, 128, 16, 128, 1, False), TransformerConfig(64, 128, 128, 4, 128, 3, True),
+     TransformerConfig(3, 48, 32, 1, 32, 50, True)],
+    ids=lambda c: f"{c.batch_size}x{c.seq_len}-d{c.d_model}-h{c.num_heads}-f{c.ffn_dim}-l{c.num_layers}",
+)
+@pytest.mark.parametrize("masking", ["none", "prefix", "general"])
+def test_encoder_parity_narrow_one_launch(device, cfg, masking):
+    """The one-launch forward of narrow models on sequences of up to 128
+    tokens, bit for bit the oracle: every head dim, lengths around its 16- and
+    32-token blocks, groups of 1, 2 and 4 sequences with a partial last one,
+    more layers than one launch's argument block holds, prefix masks, and
+    masks with holes and with sequences that see no key."""
+    sd, candidate = build_models(cfg, 55, device)
+    with torch.inference_mode():
+        x, mask = generate_random_case(cfg, device, torch.bfloat16, 3, 0.6 if masking == "prefix" else 0.0, 1.0)
+        if masking == "general":
+            g = torch.Generator(device=device).manual_seed(9)
+            mask = torch.rand(mask.shape, generator=g, device=device) < 0.7
+            mask[1] = False
+        outs = [candidate(x, mask) for _ in range(3)]
+        ref = encoder_forward(sd, x, mask, cfg.causal, cfg.num_heads, cfg.num_layers)
+        torch.cuda.synchronize()
+    # a query without a key: the reference's softmax is NaN there, the row's
+    # output is masked out unless the key mask excludes all of a valid query's keys
+    seen = torch.isfinite(ref.float()).all(-1)
+    for out in outs:
+        assert torch.equal(ref[seen], out[seen])
+        assert torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize(
+    "cfg",
     [TransformerConfig(1, 100, 256, 4, 512, 3, True), TransformerConfig(2, 64, 512, 8, 1024, 2, False),
      TransformerConfig(1, 256, 1024, 16, 1024, 2, True), TransformerConfig(3, 50, 2048, 16, 512, 2, False)],
     ids=["d256-ragged-causal", "d512", "d1024-256rows-causal", "d2048"],

@@ -33,6 +33,7 @@ SOURCES = (
     "attention_hd256.hip",
     "flash_attention.hip",
     "block_tail.hip",
+    "narrow_forward.hip",
     "capi.hip",
 )
 
@@ -64,6 +65,7 @@ EXTRA_FLAGS = {
     "attention_hd128.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
     "attention_hd256.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
     "flash_attention.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
+    "narrow_forward.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
 }
 
 

@@ -238,13 +238,47 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
     a.w_packed_rows = enc::gemm_prepack_rows(n, k);
   };
 
+  // Narrow models on sequences of at most 128 tokens run as one launch where
+  // that is faster; its 16-byte loads need 16-byte aligned operands.
+  const bool no_split = !enc::gemm_has_split_tail(T, D, D, cus) && !enc::gemm_has_split_tail(T, F, D, cus) &&
+                        !enc::gemm_has_split_tail(T, D, F, cus);
+  bool one_launch = exact && num_layers > 0 && enc::narrow_forward_supported(seq_len, D, H, F) &&
+                    enc::narrow_forward_faster(batch, seq_len, D, H) && no_split &&
+                    (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+  for (int64_t i = 0; one_launch && i < 12 * num_layers + 2; ++i)
+    one_launch = reinterpret_cast<uintptr_t>(weights[i]) % 16 == 0;
+  if (one_launch) {
+    enc::NarrowForward nf;
+    nf.x = static_cast<const bf16_t*>(x);
+    nf.out = static_cast<bf16_t*>(out);
+    nf.weights = weights;
+    if (final_norm) {
+      nf.final_g = static_cast<const bf16_t*>(weights[12 * num_layers]);
+      nf.final_b = static_cast<const bf16_t*>(weights[12 * num_layers + 1]);
+    }
+    nf.kv_len = kv_len;
+    nf.key_mask = key_mask;
+    nf.row_mask = row_mask;
+    nf.B = batch;
+    nf.S = seq_len;
+    nf.D = D;
+    nf.H = H;
+    nf.F = F;
+    nf.layers = num_layers;
+    nf.eps = eps;
+    nf.scale = scale;
+    nf.causal = causal != 0;
+    const hipError_t ne = enc::narrow_forward_bf16(nf, st);
+    if (ne != hipSuccess) return fail_hip(ne, "encoder narrow forward");
+    return ok();
+  }
+
   // Narrow models with up to 8192 tokens run the block tail (out_proj ..
   // ffn_out, and the next layer's norm1) as one kernel, whose 16-byte loads
   // need 16-byte aligned weights (all but the QKV projection's).
   // (With more tokens the four launches win: the fused kernel's one workgroup
   // per CU cannot hide its per-slab latency; measured on MI355X.)
-  bool tail_fused = enc::block_tail_supported(D, F) && T <= 8192 && !enc::gemm_has_split_tail(T, D, D, cus) &&
-                    !enc::gemm_has_split_tail(T, F, D, cus) && !enc::gemm_has_split_tail(T, D, F, cus);
+  bool tail_fused = enc::block_tail_supported(D, F) && T <= 8192 && no_split;
   for (int64_t layer = 0; tail_fused && layer < num_layers; ++layer)
     for (int idx = 0; idx < 12; ++idx)
       tail_fused = tail_fused && (idx == 2 || idx == 3 || reinterpret_cast<uintptr_t>(W(layer, idx)) % 16 == 0);

@@ -1474,7 +1474,36 @@ hipError_t ensure_gelu_table(hipStream_t st) {
   return e;
 }
 
+// Device addresses of the table and its flag, looked up once per device.
+struct GeluAddress {
+  const uint16_t* table = nullptr;
+  const uint32_t* ready = nullptr;
+};
+GeluAddress g_gelu_address[64];
+
 }  // namespace
+
+hipError_t gemm_gelu_table(hipStream_t st, const uint16_t** table, const uint32_t** ready) {
+  hipError_t e = ensure_gelu_table(st);
+  if (e != hipSuccess) return e;
+  int dev = 0;
+  e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
+  std::lock_guard<std::mutex> guard(g_gelu_mutex);
+  GeluAddress& at = g_gelu_address[dev];
+  if (at.ready == nullptr) {
+    void *t = nullptr, *r = nullptr;
+    e = hipGetSymbolAddress(&t, HIP_SYMBOL(g_gelu_table));
+    if (e == hipSuccess) e = hipGetSymbolAddress(&r, HIP_SYMBOL(g_gelu_ready));
+    if (e != hipSuccess) return e;
+    at.table = static_cast<const uint16_t*>(t);
+    at.ready = static_cast<const uint32_t*>(r);
+  }
+  *table = at.table;
+  *ready = at.ready;
+  return hipSuccess;
+}
 
 hipError_t gemm_debug_gelu_table(int32_t ready, int32_t entry, int32_t value, hipStream_t st) {
   hipError_t e = ensure_gelu_table(st);

@@ -138,6 +138,34 @@ bool block_tail_supported(int64_t d_model, int64_t ffn_dim);
 hipError_t block_tail_bf16(const BlockTailArgs& args, int64_t rows, int64_t d_model, int64_t ffn_dim, float eps,
                            int num_cus, hipStream_t stream);
 
+// Whole forward of a narrow model in one launch (per kNarrowMaxLayers layers):
+// d_model and ffn_dim of 32, 64 or 128, at most 128 tokens a sequence, the
+// attention's head dims up to 128.  weights: 12 pointers per layer in the C
+// ABI's order, each 16-byte aligned; final_g / final_b null skip the final
+// norm.  Bitwise the separate launches' output.
+constexpr int kNarrowMaxLayers = 24;
+struct NarrowForward {
+  const bf16_t* x = nullptr;
+  bf16_t* out = nullptr;
+  const void* const* weights = nullptr;
+  const bf16_t* final_g = nullptr;
+  const bf16_t* final_b = nullptr;
+  const int32_t* kv_len = nullptr;
+  const uint8_t* key_mask = nullptr;
+  const uint8_t* row_mask = nullptr;
+  int64_t B = 0, S = 0, D = 0, H = 0, F = 0, layers = 0;
+  float eps = 0.f, scale = 0.f;
+  bool causal = false;
+};
+bool narrow_forward_supported(int64_t S, int64_t D, int64_t H, int64_t F);
+// Whether that launch is the faster one for a supported shape.
+bool narrow_forward_faster(int64_t B, int64_t S, int64_t D, int64_t H);
+hipError_t narrow_forward_bf16(const NarrowForward& f, hipStream_t stream);
+
+// Device addresses of the current device's GELU table (65536 bf16) and its
+// ready flag, after enqueueing the fill on the stream if this device has none.
+hipError_t gemm_gelu_table(hipStream_t stream, const uint16_t** table, const uint32_t** ready);
+
 // Sequence lengths whose softmax summation order is reproduced exactly, and
 // whose per-head K and V^T the exact kernel's 32-bit tile offsets reach.
 bool attention_seq_supported(int64_t seq_len, int64_t head_dim);
