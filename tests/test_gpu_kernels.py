@@ -255,6 +255,25 @@ def test_linear_narrow_and_d128_shapes_bitwise(device, m, n, k):
     assert torch.equal(out[mask], (res + ref)[mask]) and torch.equal(out[~mask], res[~mask])
 
 
+@pytest.mark.parametrize(
+    "b,s,d,h",
+    [(64, 125, 1024, 4), (3, 777, 1024, 16), (300, 7, 1024, 16), (2100, 1, 512, 8), (1, 2049, 512, 8), (5, 129, 576, 9),
+     (90, 23, 1024, 128), (41, 50, 2048, 16)],
+)
+def test_qkv_ragged_sequences_bitwise(device, b, s, d, h):
+    """The ring kernel's V^T of sequences that are no whole number of 8-row
+    groups, on every tile: groups cut by a tile's edge, sequences shorter than
+    a group and than a tile's stride, many sequences a tile, one a grid."""
+    g = torch.Generator(device=device).manual_seed(b + s + d)
+    x = torch.randn(b, s, d, generator=g, device=device).bfloat16()
+    w = (torch.randn(3 * d, d, generator=g, device=device) / math.sqrt(d)).bfloat16()
+    bias = (torch.randn(3 * d, generator=g, device=device) * 0.05).bfloat16()
+    out = native.qkv_proj(x, w, bias, h)
+    for i, got in enumerate(out):
+        y = F.linear(x, w[i * d:(i + 1) * d], bias[i * d:(i + 1) * d]).view(b, s, h, d // h).transpose(1, 2)
+        assert torch.equal(y, got if i < 2 else got[..., :s].transpose(-1, -2))
+
+
 @pytest.mark.parametrize("m,n,k", [(128, 512, 2048), (64, 512, 2048), (256, 512, 2048), (16, 1536, 512), (1, 512, 512), (16, 1024, 4096), (128, 1024, 4096)])
 def test_linear_split_k_order_bitwise(device, m, n, k):
     """Shapes where torch's bf16 nn.Linear splits K: the kernel's partial sums

@@ -1083,59 +1083,56 @@ gemm_big_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int 
         off = wrap ? off + batch_stride - S : off;
       }
     }
-    // V^T otherwise: one channel, 8 consecutive rows.  Thread t owns channel
-    // t % BN of the tile and row groups t / BN, t / BN + kVStep, ... of 8 rows
-    // each.
-    static_assert(kThreads % BN == 0, "one channel per thread");
-    constexpr int kVStep = kThreads / BN;
-    const int cl = tid % BN;
-    const int vcol = n0 + cl;
-    if (!v_fast && vcol / D == 2) {
-      const int h = (vcol - 2 * D) / hd;
-      const int d = (vcol - 2 * D) - h * hd;
+    // V^T otherwise (a partial tile, or sequences that are no whole number of
+    // 8-row groups): the groups follow the sequences instead of the tile's
+    // rows, eight positions from a multiple of 8 on, so that a group is one
+    // 16-byte store again.  Group v covers positions 8 (v % G) .. of sequence
+    // v / G, G = ld_vt / 8; a sequence's last one may run into its padding
+    // columns, which nobody reads; only the groups that the tile's first and
+    // last row cut are stored by element.  (Every element by itself, with a
+    // division each, as groups of tile rows have to be: 8000x3072x1024, S = 125,
+    // 122 us against 64.5.)
+    if (!v_fast && (n0 + cp) / D == 2) {
+      const int h = (n0 + cp - 2 * D) / hd;
+      const int d = (n0 + cp - 2 * D) - h * hd;
       bf16_t* vrow = ep.v_t + (static_cast<int64_t>(h) * hd + d) * ep.ld_vt;
       const int64_t batch_stride = static_cast<int64_t>(ep.num_heads) * hd * ep.ld_vt;
-      // 8-row groups that never straddle a sequence and land 16-byte aligned
-      if (full && (S & 7) == 0 && (ep.ld_vt & 7) == 0 && 8 * kVStep <= S) {
-        int b, s;
-        locate(m0 + (tid / BN) * 8, b, s);
-        int64_t off = b * batch_stride + s;
-        for (int g = tid / BN; g < BM / 8; g += kVStep) {
-          const int r8 = g * 8;
-          uint32_t p[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            p[e] = static_cast<uint32_t>(sc[(r8 + 2 * e) * T::kLdc + cl]) |
-                   (static_cast<uint32_t>(sc[(r8 + 2 * e + 1) * T::kLdc + cl]) << 16);
-          *reinterpret_cast<u32x4*>(vrow + off) = u32x4{p[0], p[1], p[2], p[3]};
-          s += 8 * kVStep;
-          off += 8 * kVStep;
-          const bool wrap = s >= S;
-          s = wrap ? s - S : s;
-          off = wrap ? off + batch_stride - S : off;
+      const int groups = ep.ld_vt / 8;
+      const int last = min(m0 + BM, M) - 1;
+      int b, s, b_end, s_end;
+      locate(m0, b, s);
+      locate(last, b_end, s_end);
+      int sg = s / 8 + tid / kVPairs;  // this thread's first group of sequence b
+      for (;;) {
+        while (sg >= groups) {
+          sg -= groups;
+          ++b;
         }
-      } else {
-        for (int g = tid / BN; g < BM / 8; g += kVStep) {
-          const int r8 = g * 8;
-          const int row0 = m0 + r8;
-          if (row0 >= M) break;
-          int b0, s0;
-          locate(row0, b0, s0);
-          if (row0 + 7 < M && s0 + 7 < S && (s0 & 7) == 0 && (ep.ld_vt & 7) == 0) {
-            uint32_t p[4];
+        if (b > b_end || (b == b_end && sg > s_end / 8)) break;
+        const int row0 = b * S + 8 * sg - m0;              // tile row of the group's first position
+        const int rows = min(8, S - 8 * sg);
+        bf16_t* dst = vrow + b * batch_stride + 8 * sg;
+        if (row0 >= 0 && row0 + rows - 1 + m0 <= last) {
+          uint32_t w[8];  // position e: channel cp in the low half, cp + 1 in the high half
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              p[e] = static_cast<uint32_t>(sc[(r8 + 2 * e) * T::kLdc + cl]) |
-                     (static_cast<uint32_t>(sc[(r8 + 2 * e + 1) * T::kLdc + cl]) << 16);
-            *reinterpret_cast<u32x4*>(vrow + b0 * batch_stride + s0) = u32x4{p[0], p[1], p[2], p[3]};
-          } else {
-            for (int e = 0; e < 8 && row0 + e < M; ++e) {
-              int b, s;
-              locate(row0 + e, b, s);
-              vrow[b * batch_stride + s] = sc[(r8 + e) * T::kLdc + cl];
-            }
+          for (int e = 0; e < 8; ++e)
+            w[e] = *reinterpret_cast<const uint32_t*>(sc + (row0 + min(e, rows - 1)) * T::kLdc + cp);
+          u32x4 lo, hi;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            lo[e] = __builtin_amdgcn_perm(w[2 * e + 1], w[2 * e], 0x05040100u);
+            hi[e] = __builtin_amdgcn_perm(w[2 * e + 1], w[2 * e], 0x07060302u);
+          }
+          *reinterpret_cast<u32x4*>(dst) = lo;
+          *reinterpret_cast<u32x4*>(dst + ep.ld_vt) = hi;
+        } else {
+          for (int e = 0; e < rows; ++e) {
+            if (row0 + e < 0 || row0 + e + m0 > last) continue;
+            dst[e] = sc[(row0 + e) * T::kLdc + cp];
+            dst[ep.ld_vt + e] = sc[(row0 + e) * T::kLdc + cp + 1];
           }
         }
+        sg += kVStep2;
       }
     }
   }
@@ -1922,8 +1919,9 @@ hipError_t gemm_bf16_plain(const bf16_t* A, const bf16_t* W, int64_t M, int64_t 
   if (split == 2 && chunk == 128) return launch_split<2, 128>(A, W, m, n, k, epi, ep, stream);
   const bool ep_overlaps = epi == kEpiBiasGelu;
   // The large-tile head-major epilogue stores 8 channels of one head at a
-  // time (Q, K) and channel pairs (V^T): head_dim must be a multiple of 8.
-  const bool big_ok = epi != kEpiQkvHeadMajor || ep.head_dim % 8 == 0;
+  // time (Q, K) and channel pairs (V^T, in 16-byte pieces of its rows):
+  // head_dim and ld_vt must be multiples of 8.
+  const bool big_ok = epi != kEpiQkvHeadMajor || (ep.head_dim % 8 == 0 && ep.ld_vt % 8 == 0);
   switch (big_ok ? pick_big_tile(M, N, A, W, ep, ep_overlaps, num_cus) : 0) {
     case 256129: return launch_big<256, 128, 32, 3, 2>(A, W, m, n, k, epi, ep, stream);
     // 256x256 tiles: from the plain nn.Linear weight, 64-deep K blocks in two
