@@ -255,6 +255,31 @@ def test_linear_narrow_and_d128_shapes_bitwise(device, m, n, k):
     assert torch.equal(out[mask], (res + ref)[mask]) and torch.equal(out[~mask], res[~mask])
 
 
+@pytest.mark.parametrize("packed", [False, True], ids=["plain", "packed"])
+@pytest.mark.parametrize(
+    "m,n,k",
+    [(257, 64, 64), (300, 192, 192), (1000, 1024, 1024), (512, 1088, 128), (2048, 1024, 64),  # 64 x 64 tiles
+     (777, 4096, 256), (1025, 2176, 512), (1500, 4096, 512), (1537, 4096, 192), (2331, 2048, 512)],  # past them
+)
+def test_linear_ring_tiles_bitwise(device, m, n, k, packed):
+    """The ring kernel's smaller tiles (64 x 64 up to two per CU, then 128 x
+    128 with one or two per CU and 256 x 128): one K block and more, ragged
+    last rows, every epilogue, both weight layouts, bit for bit torch."""
+    if packed and native.prepack_rows(n, k) == 0:
+        pytest.skip("no packed form")
+    a, w, bias, res, _ = _linear_case(device, m, n, k, 31 * m + n + k)
+    wp = native.prepack_weight(w) if packed else None
+    ref = F.linear(a, w, bias)
+    assert torch.equal(native.linear(a, w, bias, native.ENC_EPI_BIAS, packed_weight=wp), ref)
+    assert torch.equal(native.linear(a, w, bias, native.ENC_EPI_BIAS_GELU, packed_weight=wp),
+                       F.gelu(ref, approximate="none"))
+    mask = torch.rand(m, device=device) > 0.3
+    out = native.linear(a, w, bias, native.ENC_EPI_BIAS_RESIDUAL_ZERO, residual=res, row_mask=mask, packed_weight=wp)
+    assert torch.equal(out[mask], (res + ref)[mask]) and torch.all(out[~mask] == 0)
+    out = native.linear(a, w, bias, native.ENC_EPI_BIAS_RESIDUAL_KEEP, residual=res, row_mask=mask, packed_weight=wp)
+    assert torch.equal(out[mask], (res + ref)[mask]) and torch.equal(out[~mask], res[~mask])
+
+
 @pytest.mark.parametrize(
     "b,s,d,h",
     [(64, 125, 1024, 4), (3, 777, 1024, 16), (300, 7, 1024, 16), (2100, 1, 512, 8), (1, 2049, 512, 8), (5, 129, 576, 9),

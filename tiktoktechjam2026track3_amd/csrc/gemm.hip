@@ -402,7 +402,7 @@ gemm_narrow_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, i
 }
 
 // ---------------------------------------------------------------------------
-// Large-tile kernel: BM x BN output tile (256x256, 256x128 or 128x128), four
+// Ring kernel: BM x BN output tile (256x256, 256x128, 128x128 or 64x64), four
 // wavefronts in a 2 x 2 grid, each owning a (BM/2) x (BN/2) sub-tile of 32x32
 // fp32 accumulator blocks (up to 256 registers per lane, held in AGPRs).
 //
@@ -668,10 +668,15 @@ gemm_big_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int 
     const bf16_t* rs = smem + rstage * T::kStage;
     const int slot = ((2 * rks + lhi) ^ swz) * 8;
     bf16_t* sa = smem + lstage * T::kStage;
+    // (tiles with fewer MFMAs than fragment reads a step end with reads alone)
+    constexpr int kQ = RM * RN > RM + RN ? RM * RN : RM + RN;
+    static_assert(kQ >= kPer, "a step's loads go out beside its MFMAs and reads");
 #pragma unroll
-    for (int q = 0; q < RM * RN; ++q) {
+    for (int q = 0; q < kQ; ++q) {
       const int i = q / RN, j = q % RN;
-      if constexpr (!kM16) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+      if constexpr (!kM16) {
+        if (q < RM * RN) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+      }
       if (read && q < RM) an[q] = *reinterpret_cast<const bf16x8*>(rs + a_off + q * 32 * BK + slot);
       if (read && q >= RM && q < RM + RN)
         bn[q - RM] = *reinterpret_cast<const bf16x8*>(rs + b_off + (q - RM) * 32 * BK + slot);
@@ -1763,37 +1768,49 @@ hipError_t launch_tail_split(const bf16_t* A, const bf16_t* W, int M, int N, int
   return hipGetLastError();
 }
 
-// Tile of the large-tile kernel for this shape, or 0 when the small-tile
-// kernel should run: the operands must be 16-byte aligned (16-byte loads per
-// lane), the residual / outputs too (16-byte epilogue stores), and the tile
-// count should fill the device's CUs.
+// Tile of the ring kernel for this shape, or 0 when the register-staged kernel
+// should run: the operands must be 16-byte aligned (16-byte loads per lane),
+// the residual / outputs too (16-byte epilogue stores).
 int pick_big_tile(int64_t M, int64_t N, const bf16_t* A, const bf16_t* W, const GemmEpilogueArgs& ep,
                   bool ep_overlaps, int num_cus) {
   auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (!al(A) || !al(W) || !al(ep.out) || !al(ep.residual) || !al(ep.q) || !al(ep.k) || !al(ep.v_t) ||
       !al(ep.w_packed) || reinterpret_cast<uintptr_t>(ep.bias) % 8 != 0)  // 8-byte bias loads
     return 0;
-  if (M < 1024) return 0;
-  const int64_t t256x128 = ((M + 255) / 256) * (N / 128);
-  // With two resident 256x128 tiles per CU one tile's epilogue overlaps the
-  // other's MFMA loop (when there are tiles for two per CU: a narrow N leaves
-  // most CUs idle).  It pays where the epilogue is long against the K loop:
-  // the GELU (32768x4096x1024: 314 vs 366 us on 256x256 tiles).  The
-  // residual epilogues run as fast or faster on the 256x256 tiles
-  // (32768x1024x1024 plain weight: 73.5 vs 83.2 us; 409600x1024x1024 packed:
-  // 932 vs 1007 us).
-  if (ep_overlaps && N % 128 == 0 && t256x128 >= 2 * num_cus) return 256129;
+  auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * (N / bn); };
+  // At most two 64x64 tiles per CU: the smallest tile, a four-stage ring and
+  // two workgroups per CU hide most of the latency that bounds these products.
+  // (us, before / 64x64 / 128x128: 1000x1024x1024 14.6 / 6.6 / 9.3,
+  // 512x1024x4096 68.5 / 15.4 / 27.4, 1500x1024x1024 9.4 / 8.3 / 9.5, 300x4096x1024
+  // 15.2 / 8.2 / 9.6, 4096x512x512 7.1 / 6.3 / 7.0; with more tiles 128x128 is
+  // faster: 777x4096x1024 19.4 / 14.6 / 11.3, 2331x1024x1024 10.3 / 13.1 / 10.2.)
+  if (N % 64 == 0 && tiles(64, 64) <= 2 * num_cus) return 64064;
+  if (N % 128 != 0) return 0;
+  // With two resident tiles per CU one tile's epilogue overlaps the other's
+  // MFMA loop.  It pays where the epilogue is long against the K loop, the
+  // GELU: 256x128 tiles when there are two for every CU (32768x4096x1024: 314
+  // vs 366 us on 256x256 tiles), else 128x128 tiles when there is more than
+  // one (2331x4096x1024: 36.8 vs 45.1 us, 1500x4096x1024 22.2 vs 28.2,
+  // 8000x2048x2048 81.5 vs 89.5).  The residual epilogues run as fast or faster
+  // on the 256x256 tiles (32768x1024x1024 plain weight: 73.5 vs 83.2 us;
+  // 409600x1024x1024 packed: 932 vs 1007 us).
+  if (ep_overlaps && tiles(256, 128) >= 2 * num_cus) return 256129;
+  if (ep_overlaps && tiles(128, 128) > num_cus) return 128129;
   // Whole rounds of tiles over the CUs times the tile's work, over its
-  // measured per-tile efficiency (256x128 tiles run ~10% below 256x256).
+  // efficiency: one full round at K = 1024 takes 34.5, 20.9 and 11.7 us on
+  // 256x256, 256x128 and 128x128 tiles, and several rounds of 128x128 tiles
+  // slow each other (9000x2048x2048: 5 rounds 88.8 us, 3 of 256x128 84.9).
+  // (2331x2048x2048, where 128x128 tiles need
+  // a second round: 33.5 -> 25.5 us on 256x128; 1500x4096x1024 20.4 -> 17.3;
+  // QKV 2048x3072x1024 24.2 -> 20.8.)
   auto cost = [&](int bm, int bn, double eff) {
-    const int64_t tiles = ((M + bm - 1) / bm) * (N / bn);
-    const int64_t rounds = (tiles + num_cus - 1) / num_cus;
+    const int64_t rounds = (tiles(bm, bn) + num_cus - 1) / num_cus;
     return static_cast<double>(rounds) * bm * bn / eff;
   };
-  if (N % 256 == 0 && cost(256, 256, 1.0) <= cost(256, 128, 0.9)) return 256256;
-  if (N % 128 == 0 && t256x128 >= num_cus) return 256128;
-  if (N % 128 == 0) return 128128;
-  return 0;
+  const double c256 = N % 256 == 0 ? cost(256, 256, 1.0) : 1e30;
+  const double c128 = cost(256, 128, 0.83), c64 = cost(128, 128, 0.68);
+  if (c256 <= c128 && c256 <= c64) return 256256;
+  return c128 <= c64 ? 256128 : 128128;
 }
 
 }  // namespace
@@ -1933,6 +1950,8 @@ hipError_t gemm_bf16_plain(const bf16_t* A, const bf16_t* W, int64_t M, int64_t 
       return launch_big<256, 256, 64, 2>(A, W, m, n, k, epi, ep, stream);
     case 256128: return launch_big<256, 128, 64, 3>(A, W, m, n, k, epi, ep, stream);
     case 128128: return launch_big<128, 128, 64, 3>(A, W, m, n, k, epi, ep, stream);
+    case 128129: return launch_big<128, 128, 64, 2, 2>(A, W, m, n, k, epi, ep, stream);
+    case 64064: return launch_big<64, 64, 64, 4, 2>(A, W, m, n, k, epi, ep, stream);
     default: break;
   }
   int bm, bn;
