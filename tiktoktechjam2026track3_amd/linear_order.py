@@ -199,7 +199,8 @@ def register(order: LinearOrder, device: torch.device) -> None:
 def ensure(m: int, n: int, k: int, device: torch.device) -> LinearOrder:
     """The order of [m, k] x [n, k]^T on ``device``: measured and registered on
     first use, cached for the process."""
-    device = torch.device(device)
+    if not isinstance(device, torch.device):
+        device = torch.device(device)
     index = device.index if device.index is not None else torch.cuda.current_device()
     key = (index, m, n, k)
     order = _orders.get(key)
@@ -218,8 +219,10 @@ def ensure(m: int, n: int, k: int, device: torch.device) -> LinearOrder:
 def ensure_encoder(tokens: int, d_model: int, ffn_dim: int, device: torch.device) -> List[LinearOrder]:
     """Orders of the encoder's three product shapes: q/k/v/out_proj
     [T, D] x [D, D]^T, ffn_in [T, D] x [F, D]^T and ffn_out [T, F] x [D, F]^T."""
-    shapes = {(tokens, d_model, d_model), (tokens, ffn_dim, d_model), (tokens, d_model, ffn_dim)}
-    return [ensure(m, n, k, device) for m, n, k in sorted(shapes)]
+    if d_model == ffn_dim:
+        return [ensure(tokens, d_model, d_model, device)]
+    return [ensure(tokens, d_model, d_model, device), ensure(tokens, ffn_dim, d_model, device),
+            ensure(tokens, d_model, ffn_dim, device)]
 
 
 def known_encoder_orders(tokens: int, d_model: int, ffn_dim: int, device: torch.device) -> List[LinearOrder]:
