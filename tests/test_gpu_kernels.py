@@ -729,6 +729,47 @@ def test_attention_head_dims_bitwise(device, hd, b, h, s, causal, prefix, exact)
         assert torch.equal(out[:, 0, :].view(b, h, hd), v[:, :, 0, :])
 
 
+@pytest.mark.parametrize(
+    "hd,b,h,s,causal,mask_kind,q_gain",
+    [(32, 172, 1, 257, True, "none", 1.0), (32, 64, 4, 777, False, "prefix", 1.0), (32, 32, 4, 500, True, "bytes", 8.0),
+     (32, 4, 8, 2048, True, "none", 1.0), (8, 32, 8, 320, True, "prefix", 1.0), (8, 16, 4, 1000, False, "bytes", 1.0),
+     (256, 1, 1, 129, True, "none", 1.0), (256, 2, 3, 777, False, "prefix", 4.0), (256, 1, 2, 2048, True, "bytes", 1.0),
+     (256, 64, 4, 257, True, "none", 1.0), (256, 40, 4, 500, False, "bytes", 1.0)],
+)
+def test_attention_streamed_rows_other_head_dims(device, hd, b, h, s, causal, mask_kind, q_gain):
+    """Streamed rows (head dims 8 and 32 past 256 keys in grids that fill the
+    chip: four wavefronts per SIMD, half-tile sweeps; head dim 256 past 128
+    keys: four wavefronts per 128 queries in grids of any size), at one key
+    past the resident rows, ragged last tiles, the longest rows, each mask and
+    the IEEE division path (q_gain).  Head dim 256 and power-of-32 lengths give
+    the oracle's bits; for head dims 8 and 32 the reference's P.V product
+    reduces K in another order at some lengths, and those are held to the
+    strict gate and the 99.9% bitwise share of the head-dim test above."""
+    q, k, v, v_t = _attention_inputs(device, b, h, s, 7 * s + hd + b, hd=hd)
+    q = (q.float() * q_gain).bfloat16()
+    g = torch.Generator(device=device).manual_seed(s + hd)
+    kv_len = key_mask = mask = None
+    if mask_kind == "prefix":
+        lengths = torch.randint(max(1, s // 2), s + 1, (b,), generator=g, device=device)
+        mask = torch.arange(s, device=device)[None, :] < lengths[:, None]
+        kv_len = lengths.int()
+    elif mask_kind == "bytes":
+        mask = torch.rand(b, s, generator=g, device=device) < 0.8
+        mask[:, 0] = True
+        key_mask = mask
+    out = native.attention(q, k, v_t, hd**-0.5, causal, kv_len=kv_len, key_mask=key_mask)
+    ref = _oracle_context(q, k, v, causal, mask)
+    valid = torch.ones_like(out, dtype=torch.bool)
+    if mask_kind == "prefix":
+        valid = mask[..., None].expand_as(out)
+        assert torch.all(out[~valid] == 0)
+    if hd == 256:
+        assert torch.equal(ref[valid], out[valid]), f"max abs {_context_error(ref[valid], out[valid])}"
+    else:
+        assert strict_gate(ref[valid], out[valid]) == 0
+        assert bitwise_fraction(ref[valid], out[valid]) > 0.999
+
+
 def test_attention_online_rejects_other_head_dims(device):
     q, k, v, v_t = _attention_inputs(device, 1, 1, 64, 3, hd=32)
     with pytest.raises(native.EncoderKernelError, match="head_dim must be 64"):

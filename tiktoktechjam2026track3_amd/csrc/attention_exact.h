@@ -124,7 +124,8 @@ __device__ __forceinline__ int tile_key(int kb32, int r, int h) {
 // bound).  Long head-dim-64 rows with at least four workgroups per CU use 4
 // (at most 128 VGPRs, a few spilled; see dispatch_order); most head-dim-64
 // short rows use 3 with the half-tile sweeps (kHalfTiles: at most 168
-// VGPRs, see dispatch_order).
+// VGPRs), head dims 8 and 32 use 4 with them (at most 126 VGPRs, see
+// dispatch_order).
 template <int HD, int NW, bool CAUSAL, int MASK, bool POW2_SCALE, bool BLOCK_ORDER, int RES, int OCC>
 __global__ void __launch_bounds__(NW * kWave, OCC)
 attn_fwd_kernel(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ Kg,
@@ -137,12 +138,12 @@ attn_fwd_kernel(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ Kg,
   // short-row regime with a power-of-two scale: gaps stay unscaled, the scale
   // folds into expf's constants (exp_gap below)
   constexpr bool kFoldScale = POW2_SCALE && !BLOCK_ORDER;
-  // Short rows streamed through the ring at three wavefronts per SIMD: sweeps
-  // B and C work on one 32-key half of a tile at a time, so that half of the
-  // scores, weights and P fragments are live at once (at most 168 VGPRs
-  // instead of 250, none spilled).  Same MFMA chains and per-score operations
+  // Short rows streamed through the ring at three or four wavefronts per SIMD:
+  // sweeps B and C work on one 32-key half of a tile at a time, so that half
+  // of the scores, weights and P fragments are live at once (head dim 64: at
+  // most 168 VGPRs instead of 250, a masked form spills two).  Same MFMA chains and per-score operations
   // in the same order, so the same bits.
-  constexpr bool kHalfTiles = !BLOCK_ORDER && RES == 0 && OCC == 3;
+  constexpr bool kHalfTiles = !BLOCK_ORDER && RES == 0 && OCC >= 3;
   constexpr int kThreads = NW * kWave;
   constexpr int kBQ = kSplit ? 32 : NW * 32;
   constexpr int kTileElems = kBKV * HD;  // one K or V^T tile, bf16 elements
@@ -274,7 +275,7 @@ attn_fwd_kernel(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ Kg,
     v_voff[j] = static_cast<int>((static_cast<uint32_t>(rv) * static_cast<uint32_t>(ld_vt) +
                                   static_cast<uint32_t>(((lane & 7) ^ v_swz(rv)) * 8)) * 2u);
   }
-  auto issue_full = [&](int buf, int k0, bool with_v) {
+  auto issue_full = [&](int buf, int k0, bool with_v) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < kLoadsPerWave; ++j) {
       const int slab = NW * j + wave;
@@ -329,8 +330,12 @@ attn_fwd_kernel(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ Kg,
   // wavefronts need; keeping them out of the body's loop (rather than skipping
   // the body per tile) keeps the accumulators free of per-tile register
   // copies.  With resident tiles the body reads tile t from buffer t.
+  // (The sweeps and their bodies are inlined by attribute: the compiler left
+  // head dim 256's as calls, with the context accumulators, Q fragments and
+  // load offsets in scratch memory, 736 and 1248 bytes a lane; see
+  // dispatch_order.)
   bool resident = false;
-  auto sweep = [&](auto next, bool with_v, int active, auto body) {
+  auto sweep = [&](auto next, bool with_v, int active, auto body) __attribute__((always_inline)) {
     if (RES > 0) {
       if (!resident) {
         for (int t = 0; t < nkb; ++t) issue_tile(t, t, true);
@@ -389,7 +394,7 @@ attn_fwd_kernel(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ Kg,
   const int active = CAUSAL ? min(nkb, wq_last / kBKV + 1) : nkb;
 
   // Raw fp32 dot products of the 64-key tile in LDS buffer `buf`.
-  auto tile_dots = [&](int buf, f32x16 (&s)[2]) {
+  auto tile_dots = [&](int buf, f32x16 (&s)[2]) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       s[0][r] = 0.f;
@@ -488,7 +493,7 @@ attn_fwd_kernel(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ Kg,
     }
   };
   auto vmin = [](float a, float b) { return fminf(a, b); };
-  auto max_body = [&](int buf, int kb, f32x16 (&s)[2]) {
+  auto max_body = [&](int buf, int kb, f32x16 (&s)[2]) __attribute__((always_inline)) {
     const int k0 = kb * kBKV;
     tile_dots(buf, s);
     if (tile_needs_mask(k0)) {
@@ -799,7 +804,7 @@ attn_fwd_kernel(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ Kg,
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
   // s holds the gaps, or (have_e) the weights e themselves
-  auto make_pf = [&](f32x16 (&s)[2], bool have_e, bf16x8 (&pf)[4]) {
+  auto make_pf = [&](f32x16 (&s)[2], bool have_e, bf16x8 (&pf)[4]) __attribute__((always_inline)) {
     if (BLOCK_ORDER || !slow_div) {
 #pragma unroll
       for (int kb32 = 0; kb32 < 2; ++kb32) {
@@ -828,7 +833,7 @@ attn_fwd_kernel(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ Kg,
       }
     }
   };
-  auto pv_mfma = [&](int buf, const bf16x8 (&pf)[4]) {
+  auto pv_mfma = [&](int buf, const bf16x8 (&pf)[4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
 #pragma unroll
@@ -839,7 +844,7 @@ attn_fwd_kernel(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ Kg,
       }
     }
   };
-  auto pv_body = [&](int buf, f32x16 (&s)[2], bool have_e) {
+  auto pv_body = [&](int buf, f32x16 (&s)[2], bool have_e) __attribute__((always_inline)) {
     bf16x8 pf[4];
     make_pf(s, have_e, pf);
     pv_mfma(buf, pf);
@@ -1027,7 +1032,16 @@ hipError_t dispatch_order(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf
       if (S <= 4 * kBKV)
         return launch_attn<HD, 1, CAUSAL, MASK, POW2, false, 4>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
     }
-    return launch_attn<HD, 1, CAUSAL, MASK, POW2, false>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
+    // Head dim 256 keeps four wavefronts however small the grid: its K and V^T
+    // ring takes 128 KiB, so a CU holds one workgroup, and one wavefront's
+    // load offsets for whole tiles leave the registers (480 bytes of scratch).
+    // 4 sequences x 4 heads of 1024 causal keys 1223 us (the bodies called,
+    // see sweep) -> 825 one wavefront inlined -> 109 four wavefronts; 1 x 4 x
+    // 200 274 -> 197 -> 36; 64 x 4 x 500 causal (four wavefronts before, too)
+    // 1170 -> 209.
+    if constexpr (HD < 256)
+      return launch_attn<HD, 1, CAUSAL, MASK, POW2, false>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
+    return launch_attn<HD, 4, CAUSAL, MASK, POW2, false>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
   }
   if (S <= 2 * kBKV)
     return launch_attn<HD, 4, CAUSAL, MASK, POW2, false, 2>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
@@ -1048,6 +1062,13 @@ hipError_t dispatch_order(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf
     if (CAUSAL || S > 512)
       return launch_attn<HD, 4, CAUSAL, MASK, POW2, false, 0, 3>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
   }
+  // Head dims 8 and 32: the softmax's per-score operations are all there is,
+  // and four wavefronts per SIMD with the half-tile sweeps hide more of their
+  // latency than two: 64 x 4 heads of 32, 1024 causal keys 175.6 -> 168.7 us,
+  // prefix 777 95.4 -> 92.7, 200 x 4 x 300 118.9 -> 116.9, byte masks level;
+  // 64 x 16 heads of 8, 1024 causal keys 557 -> 532.
+  if constexpr (HD <= 32)
+    return launch_attn<HD, 4, CAUSAL, MASK, POW2, false, 0, 4>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
   return launch_attn<HD, 4, CAUSAL, MASK, POW2, false>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
 }
 
