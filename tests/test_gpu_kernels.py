@@ -770,6 +770,32 @@ def test_attention_streamed_rows_other_head_dims(device, hd, b, h, s, causal, ma
         assert bitwise_fraction(ref[valid], out[valid]) > 0.999
 
 
+@pytest.mark.parametrize(
+    "hd,b,h,s,causal",
+    [(256, 16, 4, 128, True), (256, 17, 4, 97, True), (128, 32, 2, 128, False), (128, 33, 2, 125, True),
+     (64, 16, 8, 128, True), (64, 17, 8, 125, True), (32, 32, 8, 128, False), (32, 33, 8, 128, True),
+     (8, 48, 8, 125, True), (8, 49, 8, 125, False), (128, 8, 4, 256, False), (128, 9, 4, 256, False),
+     (128, 1, 4, 200, True), (64, 8, 8, 256, True), (64, 9, 8, 256, True), (64, 1, 4, 193, True),
+     (32, 16, 8, 256, False), (32, 17, 8, 256, False), (32, 1, 4, 257, True), (64, 2, 8, 2048, False),
+     (64, 3, 8, 2048, False), (64, 1, 4, 300, True), (128, 2, 8, 1024, True), (128, 3, 8, 1024, True),
+     (128, 1, 2, 1000, False)],
+)
+def test_attention_small_and_full_workgroups_bitwise(device, hd, b, h, s, causal):
+    """Both sides of the rule that gives small problems workgroups of 32
+    queries: the largest grids that fit the chip at once and the first past
+    them, for the key split, the resident and the streamed rows, and rows that
+    end inside a tile.  The oracle's bits (head dims 8 and 32: strict gate and
+    a 99.9% bitwise share past 128 keys, as in the head-dim test above)."""
+    q, k, v, v_t = _attention_inputs(device, b, h, s, 3 * s + hd + b, hd=hd)
+    out = native.attention(q, k, v_t, hd**-0.5, causal)
+    ref = _oracle_context(q, k, v, causal, None)
+    if hd >= 64 or s <= 128:
+        assert torch.equal(ref, out), f"max abs {_context_error(ref, out)}"
+    else:
+        assert strict_gate(ref, out) == 0
+        assert bitwise_fraction(ref, out) > 0.999
+
+
 def test_attention_online_rejects_other_head_dims(device):
     q, k, v, v_t = _attention_inputs(device, 1, 1, 64, 3, hd=32)
     with pytest.raises(native.EncoderKernelError, match="head_dim must be 64"):

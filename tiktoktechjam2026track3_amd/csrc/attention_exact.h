@@ -1016,32 +1016,50 @@ hipError_t dispatch_order(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf
     }
     return launch_attn<HD, 4, CAUSAL, MASK, POW2, true>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
   }
-  // Small problems use workgroups of 32 queries (one wavefront, or two that
-  // split the keys) so more of the 256 CUs get work; larger ones share each
-  // K/V tile among 4 wavefronts.
-  // Rows of at most 256 keys keep every tile resident in LDS (at most 128 keys
-  // for head dim 256, whose four resident tiles would exceed the 160 KiB of
-  // LDS of a CU).
+  // Workgroups of 32 queries (one wavefront, or two that split the keys) give
+  // small problems more of the 256 CUs; larger ones share each K/V tile among
+  // 4 wavefronts.  Rows of at most 256 keys keep every tile resident in LDS
+  // (at most 128 keys for head dim 256, whose four resident tiles would exceed
+  // the 160 KiB of LDS of a CU).
+  //
+  // The small workgroups are taken while all of them fit the chip at once,
+  // that is LDS bytes into 160 KiB per CU: past that the second round costs
+  // what the first did.  Measured, small / 4 wavefronts, us, at rows of 125
+  // keys with a prefix mask: head dim 256 (one per CU) 64 x 4 51.3 / 24.5, 32
+  // x 4 29.3 / 21.1, 16 x 4 17.6 / 18.2; 128 (one) 32 x 8 31.6 / 13.9, 8 x 8
+  // 11.9 / 12.4; 64 (two) 48 x 8 21.4 / 13.0; 32 (four) 48 x 8 14.0 / 10.9.
+  // Resident tiles of 200 - 256 keys: 64 31 x 8 51.2 / 24.2, 8 x 8 14.0 / 13.9;
+  // 128 16 x 8 50.0 / 22.2.  Streamed rows: 64 3 x 8 x 2048 187 / 145, 1 x 8 x
+  // 1024 47.8 / 51.2; 128 4 x 8 x 1024 146 / 75.5, 1 x 8 x 512 38.1 / 40.1.
+  // A row past 128 keys that ends inside a tile loads that tile through
+  // registers, in every sweep, which one wavefront does too slowly from the
+  // head dim on that the rule names (128 1 x 8 x 200 24.7 / 20.3, 1 x 8 x 1000
+  // 78.6 / 72.0; 64 1 x 8 x 300 23.5 / 21.3; 32 1 x 8 x 200 15.2 / 14.3, but 1
+  // x 8 x 1000 48.0 / 50.5).
+  // Head dim 256 streams its rows by four wavefronts however small the grid:
+  // its ring takes 128 KiB, and one wavefront's load offsets for whole tiles
+  // leave the registers (480 bytes of scratch).  4 x 4 heads of 1024 causal
+  // keys 1223 us (the bodies called, see sweep) -> 825 one wavefront inlined
+  // -> 109 four wavefronts; 1 x 4 x 200 274 -> 197 -> 36; 64 x 4 x 500 causal
+  // (four wavefronts before, too) 1170 -> 209.
   constexpr bool kRes4 = attn_lds_bytes(HD, 4) <= 160 * 1024;
   const int64_t groups128 = static_cast<int64_t>(B) * H * ((S + 127) / 128);
+  const int64_t groups32 = static_cast<int64_t>(B) * H * ((S + 31) / 32);
+  auto fits = [&](size_t lds) { return groups32 <= 256 * static_cast<int64_t>(160 * 1024 / lds); };
   if (groups128 < 512) {
+    const bool whole_tiles = S % kBKV == 0 || HD == 8 || (HD == 32 && S > 4 * kBKV);
     // rows of at most 128 keys: two wavefronts per 32 queries (key split)
-    if (S <= 2 * kBKV)
-      return launch_attn<HD, 2, CAUSAL, MASK, POW2, false, 2>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
-    if constexpr (kRes4) {
-      if (S <= 4 * kBKV)
-        return launch_attn<HD, 1, CAUSAL, MASK, POW2, false, 4>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
+    if (S <= 2 * kBKV) {
+      if (fits(attn_lds_bytes(HD, 2, true)))
+        return launch_attn<HD, 2, CAUSAL, MASK, POW2, false, 2>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
+    } else if constexpr (kRes4) {
+      if (S <= 4 * kBKV) {
+        if (whole_tiles && fits(attn_lds_bytes(HD, 4)))
+          return launch_attn<HD, 1, CAUSAL, MASK, POW2, false, 4>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
+      } else if (whole_tiles && fits(attn_lds_bytes(HD, 0))) {
+        return launch_attn<HD, 1, CAUSAL, MASK, POW2, false>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
+      }
     }
-    // Head dim 256 keeps four wavefronts however small the grid: its K and V^T
-    // ring takes 128 KiB, so a CU holds one workgroup, and one wavefront's
-    // load offsets for whole tiles leave the registers (480 bytes of scratch).
-    // 4 sequences x 4 heads of 1024 causal keys 1223 us (the bodies called,
-    // see sweep) -> 825 one wavefront inlined -> 109 four wavefronts; 1 x 4 x
-    // 200 274 -> 197 -> 36; 64 x 4 x 500 causal (four wavefronts before, too)
-    // 1170 -> 209.
-    if constexpr (HD < 256)
-      return launch_attn<HD, 1, CAUSAL, MASK, POW2, false>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
-    return launch_attn<HD, 4, CAUSAL, MASK, POW2, false>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
   }
   if (S <= 2 * kBKV)
     return launch_attn<HD, 4, CAUSAL, MASK, POW2, false, 2>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
