@@ -116,9 +116,9 @@ def test_encoder_parity_narrow_ragged(device, cfg):
     "cfg",
     [TransformerConfig(3, 1, 32, 1, 64, 2, True), TransformerConfig(9, 16, 64, 2, 32, 2, False),
      TransformerConfig(5, 17, 64, 1, 128, 2, True), TransformerConfig(33, 32, 32, 4, 128, 2, False),
-     TransformerConfig(80, 33, 64, 8, 64, 2, True), TransformerConfig(16, 97, 128, 2, 128, 2, True),
-     TransformerConfig(17, 127, 128, 1, 32, 2, False), TransformerConfig(65, 112, 128, 4, 64, 2, True),
-     TransformerConfig(160, 128, 128, 16, 128, 1, False), TransformerConfig(64, 128, 128, 4, 128, 3, True),
+     TransformerConfig(180, 33, 64, 8, 64, 2, True), TransformerConfig(49, 97, 128, 2, 128, 2, True),
+     TransformerConfig(49, 127, 128, 1, 32, 2, False), TransformerConfig(97, 112, 128, 4, 64, 2, True),
+     TransformerConfig(240, 128, 128, 16, 128, 1, False), TransformerConfig(96, 128, 128, 4, 128, 3, True),
      TransformerConfig(3, 48, 32, 1, 32, 50, True)],
     ids=lambda c: f"{c.batch_size}x{c.seq_len}-d{c.d_model}-h{c.num_heads}-f{c.ffn_dim}-l{c.num_layers}",
 )
@@ -145,6 +145,46 @@ def test_encoder_parity_narrow_one_launch(device, cfg, masking):
     for out in outs:
         assert torch.equal(ref[seen], out[seen])
         assert torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize(
+    "cfg",
+    [TransformerConfig(64, 129, 128, 4, 128, 2, True), TransformerConfig(33, 259, 64, 1, 32, 2, False),
+     TransformerConfig(9, 1001, 128, 1, 64, 1, True), TransformerConfig(300, 131, 32, 1, 128, 3, True),
+     TransformerConfig(8200, 1, 128, 16, 128, 1, False), TransformerConfig(100, 100, 128, 16, 32, 2, True),
+     TransformerConfig(31, 272, 64, 2, 64, 1, True), TransformerConfig(1, 16, 128, 16, 32, 2, True),
+     TransformerConfig(2, 133, 128, 1, 128, 2, False), TransformerConfig(5, 129, 64, 8, 128, 1, True),
+     TransformerConfig(3, 700, 32, 1, 32, 2, True), TransformerConfig(8, 1000, 128, 2, 64, 2, True)],
+    ids=lambda c: f"{c.batch_size}x{c.seq_len}-d{c.d_model}-h{c.num_heads}-f{c.ffn_dim}-l{c.num_layers}",
+)
+@pytest.mark.parametrize("masking", ["none", "prefix", "general"])
+def test_encoder_parity_narrow_rows(device, cfg, masking):
+    """Narrow models that one launch does not serve: norm1 + QKV (its feature
+    blocks split among workgroups where the tokens are few) and the block tail
+    (with the final norm in the last one; past 8192 tokens by 16 tokens a
+    wavefront) around the attention.  Sequences that end inside a
+    16-token slab and inside V^T's 8-token padding, workgroups of 4, 8 and 16
+    wavefronts, every width; the oracle's bits (head dim 32 past 128 tokens:
+    the gate of the other parity tests, its P.V product reduces K in another
+    order at some lengths)."""
+    sd, candidate = build_models(cfg, 56, device)
+    with torch.inference_mode():
+        x, mask = generate_random_case(cfg, device, torch.bfloat16, 4, 0.6 if masking == "prefix" else 0.0, 1.0)
+        if masking == "general":
+            g = torch.Generator(device=device).manual_seed(9)
+            mask = torch.rand(mask.shape, generator=g, device=device) < 0.7
+            mask[:, 0] = True
+        outs = [candidate(x, mask) for _ in range(3)]
+        ref = encoder_forward(sd, x, mask, cfg.causal, cfg.num_heads, cfg.num_layers)
+        torch.cuda.synchronize()
+    exact = cfg.d_model // cfg.num_heads >= 64 or cfg.seq_len <= 128
+    for out in outs:
+        assert torch.equal(outs[0], out)
+        if exact:
+            assert torch.equal(ref, out)
+        else:
+            result = compare(ref, out, RTOL, ATOL)
+            assert result["passed"], result
 
 
 @pytest.mark.parametrize(

@@ -34,6 +34,7 @@ SOURCES = (
     "flash_attention.hip",
     "block_tail.hip",
     "narrow_forward.hip",
+    "narrow_rows.hip",
     "capi.hip",
 )
 
@@ -66,6 +67,7 @@ EXTRA_FLAGS = {
     "attention_hd256.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
     "flash_attention.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
     "narrow_forward.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
+    "narrow_rows.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
 }
 
 

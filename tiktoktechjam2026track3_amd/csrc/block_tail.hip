@@ -9,15 +9,16 @@
 // matrices fit in LDS together (104 KB at 128 / 128), so one persistent
 // workgroup per CU loads them once and walks 16-row slabs of the tokens: the
 // context and residual rows come in, every intermediate stays in LDS, and
-// only x_out goes out (with, optionally, the next layer's norm1 of the same
-// rows).  For these sizes the products are latency-bound and the launches it
-// saves per layer (three, four with the next norm1) matter more than MFMA
-// rate.
+// only x_out goes out (or, after the last layer, the final norm of it).  For
+// these sizes the products are latency-bound: eight wavefronts take one
+// 16-column block of each product, so a slab passes through three short chains
+// (four wavefronts with two blocks each and 16-deep MFMAs, the biases loaded
+// inside the chains: 9 us for 128 rows at 128 / 128 against 6).
 //
 // The arithmetic is the wide path's, operation for operation, so the output
-// is bitwise the same: each product accumulates K sequentially in 16-deep
-// MFMA steps (v_mfma_f32_16x16x16_bf16, as the skinny GEMM; the library splits
-// none of these shapes), y = bf16(acc + bias) at the nn.Linear boundary, the
+// is bitwise the same: each product accumulates K sequentially in 32-deep
+// MFMA steps (v_mfma_f32_16x16x32_bf16, the same bits as the 16-deep ones; the
+// library splits none of these shapes), y = bf16(acc + bias) at the nn.Linear boundary, the
 // residual adds and GELU-erf as in the GEMM epilogues, and norm2 through
 // packed_row_stats, the LayerNorm kernel's reduction for rows of <= 128.
 #include "common.h"
@@ -29,9 +30,8 @@ namespace enc {
 namespace {
 
 constexpr int kTailRows = 16;       // rows per slab: the MFMA M dimension
-constexpr int kTailThreads = 256;  // 4 wavefronts
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
+constexpr int kTailWaves = 8;
+constexpr int kTailThreads = kTailWaves * kWave;
 
 // LDS row stride of a K-wide operand, bf16 elements: 16 bytes of padding put
 // consecutive rows 4 banks apart, so the 16 rows of a fragment read spread
@@ -48,14 +48,14 @@ constexpr size_t tail_lds_bytes(int d, int f) {
 }
 
 // MFMA fragment of LDS row `row` (K-wide operand) at K offset k0: lane group g
-// holds k0 + 4g .. k0 + 4g + 3 (A: row = l % 16; B: row = output column).
+// holds k0 + 8g .. k0 + 8g + 7 (A: row = l % 16; B: row = output column).
 template <int K>
-__device__ __forceinline__ s16x4 tail_frag(const bf16_t* base, int row, int k0, int g) {
-  return *reinterpret_cast<const s16x4*>(base + row * tail_ld(K) + k0 + 4 * g);
+__device__ __forceinline__ bf16x8 tail_frag(const bf16_t* base, int row, int k0, int g) {
+  return *reinterpret_cast<const bf16x8*>(base + row * tail_ld(K) + k0 + 8 * g);
 }
 
 // NROWS x K bf16 row-major (global) <-> registers <-> LDS (padded stride):
-// chunk i of this thread is 16-byte chunk tid + 256 i of the matrix.  The
+// chunk i of this thread is 16-byte chunk tid + kTailThreads i of the matrix.  The
 // three weight matrices are loaded into registers together and only then
 // stored, so their loads share one memory round trip.
 template <int K, int NROWS>
@@ -86,12 +86,13 @@ block_tail_kernel(const bf16_t* __restrict__ ctx, const bf16_t* __restrict__ x, 
                   const bf16_t* __restrict__ bo, const bf16_t* __restrict__ g2, const bf16_t* __restrict__ be2,
                   const bf16_t* __restrict__ w1, const bf16_t* __restrict__ b1, const bf16_t* __restrict__ w2,
                   const bf16_t* __restrict__ b2, bf16_t* __restrict__ out, int rows, float eps,
-                  const uint8_t* __restrict__ row_mask, const bf16_t* __restrict__ g1n,
-                  const bf16_t* __restrict__ be1n, bf16_t* __restrict__ ln_out) {
+                  const uint8_t* __restrict__ row_mask, const bf16_t* __restrict__ final_g,
+                  const bf16_t* __restrict__ final_b) {
   static_assert((D == 32 || D == 64 || D == 128) && (F == 32 || F == 64 || F == 128), "d_model, ffn_dim");
   constexpr int kLdD = tail_ld(D), kLdF = tail_ld(F);
   constexpr int kSlabChunks = kTailRows * (D / 8);  // 16-byte chunks of a [16][D] slab
   static_assert(kSlabChunks <= kTailThreads, "one chunk of each slab operand per thread");
+  static_assert(D / 16 <= kTailWaves && F / 16 <= kTailWaves, "one column block per wavefront");
   extern __shared__ __attribute__((aligned(16))) bf16_t tail_lds[];
   bf16_t* sWo = tail_lds;
   bf16_t* sW1 = sWo + D * kLdD;
@@ -105,33 +106,6 @@ block_tail_kernel(const bf16_t* __restrict__ ctx, const bf16_t* __restrict__ x, 
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int l16 = lane & 15;
   const int g = lane >> 4;
-
-  {
-    using RWo = TailRows<D, D>;
-    using RW1 = TailRows<D, F>;
-    using RW2 = TailRows<F, D>;
-    u32x4 vo[RWo::kPer], v1[RW1::kPer], v2[RW2::kPer];
-    RWo::load(vo, wo, tid);
-    RW1::load(v1, w1, tid);
-    RW2::load(v2, w2, tid);
-    RWo::store(vo, sWo, tid);
-    RW1::store(v1, sW1, tid);
-    RW2::store(v2, sW2, tid);
-  }
-
-  // norm2's gamma / beta for this lane's vector (rows of D = 4 L elements)
-  constexpr int L = D / 4;
-  constexpr int R = kWave / L;  // rows per wavefront in the norm2 pass
-  const int seg = lane / L, j = lane % L;
-  const u32x2 gw = *reinterpret_cast<const u32x2*>(g2 + 4 * j);
-  const u32x2 bw = *reinterpret_cast<const u32x2*>(be2 + 4 * j);
-  // the next layer's norm1 (optional: ln_out == nullptr skips it)
-  const bool next_norm = ln_out != nullptr;
-  u32x2 gn = {0u, 0u}, bn = {0u, 0u};
-  if (next_norm) {
-    gn = *reinterpret_cast<const u32x2*>(g1n + 4 * j);
-    bn = *reinterpret_cast<const u32x2*>(be1n + 4 * j);
-  }
 
   // the slab's context and residual chunks travel in registers one slab ahead
   const int slabs = (rows + kTailRows - 1) / kTailRows;
@@ -148,6 +122,39 @@ block_tail_kernel(const bf16_t* __restrict__ ctx, const bf16_t* __restrict__ x, 
     }
   };
   fetch(blockIdx.x);
+
+  // norm2's gamma / beta for this lane's vector (rows of D = 4 L elements)
+  constexpr int L = D / 4;
+  constexpr int R = kWave / L;  // rows per wavefront in the norm2 pass
+  const int seg = lane / L, j = lane % L;
+  const u32x2 gw = *reinterpret_cast<const u32x2*>(g2 + 4 * j);
+  const u32x2 bw = *reinterpret_cast<const u32x2*>(be2 + 4 * j);
+  // the final norm's (optional)
+  const bool final_norm = final_g != nullptr;
+  u32x2 gn = {0u, 0u}, bn = {0u, 0u};
+  if (final_norm) {
+    gn = *reinterpret_cast<const u32x2*>(final_g + 4 * j);
+    bn = *reinterpret_cast<const u32x2*>(final_b + 4 * j);
+  }
+  // this lane's column of the three products and its biases (a wavefront
+  // takes one 16-column block of each; past the width, the last column's)
+  const int col = wave * 16 + l16;
+  const float bias_o = bf16_to_f32(bo[min(col, D - 1)]);
+  const float bias_1 = bf16_to_f32(b1[min(col, F - 1)]);
+  const float bias_2 = bf16_to_f32(b2[min(col, D - 1)]);
+
+  {
+    using RWo = TailRows<D, D>;
+    using RW1 = TailRows<D, F>;
+    using RW2 = TailRows<F, D>;
+    u32x4 vo[RWo::kPer], v1[RW1::kPer], v2[RW2::kPer];
+    RWo::load(vo, wo, tid);
+    RW1::load(v1, w1, tid);
+    RW2::load(v2, w2, tid);
+    RWo::store(vo, sWo, tid);
+    RW1::store(v1, sW1, tid);
+    RW2::store(v2, sW2, tid);
+  }
 
   for (int slab = blockIdx.x; slab < slabs; slab += gridDim.x) {
     const int r0 = slab * kTailRows;
@@ -171,18 +178,16 @@ block_tail_kernel(const bf16_t* __restrict__ ctx, const bf16_t* __restrict__ x, 
     __syncthreads();
 
     // ---- out_proj + residual (rows masked out keep the residual) -> sX ----
-    for (int cb = wave; cb < D / 16; cb += 4) {
+    if (wave < D / 16) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks)
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(tail_frag<D>(sA, l16, ks * 16, g),
-                                                        tail_frag<D>(sWo, cb * 16 + l16, ks * 16, g), acc, 0, 0, 0);
-      const int col = cb * 16 + l16;
-      const float bias = bf16_to_f32(bo[col]);
+      for (int ks = 0; ks < D / 32; ++ks)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tail_frag<D>(sA, l16, ks * 32, g),
+                                                        tail_frag<D>(sWo, col, ks * 32, g), acc, 0, 0, 0);
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         const int r = 4 * g + jj;
-        const float y = round_bf16(acc[jj] + bias);  // nn.Linear output boundary
+        const float y = round_bf16(acc[jj] + bias_o);  // nn.Linear output boundary
         bf16_t* px = sX + r * kLdD + col;
         const bf16_t old = *px;
         *px = keep[jj] ? f32_to_bf16(bf16_to_f32(old) + y) : old;
@@ -191,7 +196,7 @@ block_tail_kernel(const bf16_t* __restrict__ ctx, const bf16_t* __restrict__ x, 
     __syncthreads();
 
     // ---- norm2 (no row mask) -> sA ----
-    for (int p = 0; p < kTailRows; p += 4 * R) {
+    for (int p = 0; p < kTailRows; p += kTailWaves * R) {
       const int r = p + wave * R + seg;
       const int rr = r < kTailRows ? r : kTailRows - 1;  // lanes past the slab only join the shuffles
       const u32x2 w = *reinterpret_cast<const u32x2*>(sX + rr * kLdD + 4 * j);
@@ -210,49 +215,44 @@ block_tail_kernel(const bf16_t* __restrict__ ctx, const bf16_t* __restrict__ x, 
     __syncthreads();
 
     // ---- ffn_in + GELU -> sH ----
-    for (int cb = wave; cb < F / 16; cb += 4) {
+    if (wave < F / 16) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks)
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(tail_frag<D>(sA, l16, ks * 16, g),
-                                                        tail_frag<D>(sW1, cb * 16 + l16, ks * 16, g), acc, 0, 0, 0);
-      const int col = cb * 16 + l16;
-      const float bias = bf16_to_f32(b1[col]);
+      for (int ks = 0; ks < D / 32; ++ks)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tail_frag<D>(sA, l16, ks * 32, g),
+                                                        tail_frag<D>(sW1, col, ks * 32, g), acc, 0, 0, 0);
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
-        const float y = round_bf16(acc[jj] + bias);
+        const float y = round_bf16(acc[jj] + bias_1);
         sH[(4 * g + jj) * kLdF + col] = f32_to_bf16(gelu_erf(y));
       }
     }
     __syncthreads();
 
     // ---- ffn_out + residual (rows masked out become 0) -> sA ----
-    for (int cb = wave; cb < D / 16; cb += 4) {
+    if (wave < D / 16) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < F / 16; ++ks)
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(tail_frag<F>(sH, l16, ks * 16, g),
-                                                        tail_frag<F>(sW2, cb * 16 + l16, ks * 16, g), acc, 0, 0, 0);
-      const int col = cb * 16 + l16;
-      const float bias = bf16_to_f32(b2[col]);
+      for (int ks = 0; ks < F / 32; ++ks)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tail_frag<F>(sH, l16, ks * 32, g),
+                                                        tail_frag<F>(sW2, col, ks * 32, g), acc, 0, 0, 0);
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         const int r = 4 * g + jj;
-        const float y = round_bf16(acc[jj] + bias);
+        const float y = round_bf16(acc[jj] + bias_2);
         sA[r * kLdD + col] = keep[jj] ? f32_to_bf16(bf16_to_f32(sX[r * kLdD + col]) + y) : bf16_t(0);
       }
     }
     __syncthreads();
 
-    // ---- block output, 16-byte stores ----
-    if (has_chunk && r0 + my_r < rows)
-      *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(r0 + my_r) * D + my_ch * 8) =
-          *reinterpret_cast<const u32x4*>(sA + my_r * kLdD + my_ch * 8);
-
-    // ---- the next layer's norm1 of the block output rows (no row mask, as
-    // the separate launch) -> ln_out ----
-    if (next_norm) {
-      for (int p = 0; p < kTailRows; p += 4 * R) {
+    if (!final_norm) {
+      // ---- block output, 16-byte stores ----
+      if (has_chunk && r0 + my_r < rows)
+        *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(r0 + my_r) * D + my_ch * 8) =
+            *reinterpret_cast<const u32x4*>(sA + my_r * kLdD + my_ch * 8);
+    } else {
+      // ---- the final norm of the block output rows (rows masked out stay 0) ----
+      for (int p = 0; p < kTailRows; p += kTailWaves * R) {
         const int r = p + wave * R + seg;
         const int rr = r < kTailRows ? r : kTailRows - 1;  // lanes past the slab only join the shuffles
         const u32x2 w = *reinterpret_cast<const u32x2*>(sA + rr * kLdD + 4 * j);
@@ -260,12 +260,13 @@ block_tail_kernel(const bf16_t* __restrict__ ctx, const bf16_t* __restrict__ x, 
         float mean, rstd;
         packed_row_stats<L>(v, j, seg, eps, &mean, &rstd);
         if (r < kTailRows && r0 + r < rows) {
+          const bool live = row_mask == nullptr || row_mask[r0 + r] != 0;
           const float ga[4] = {lo_bf16(gn[0]), hi_bf16(gn[0]), lo_bf16(gn[1]), hi_bf16(gn[1])};
           const float be[4] = {lo_bf16(bn[0]), hi_bf16(bn[0]), lo_bf16(bn[1]), hi_bf16(bn[1])};
           float o[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = fmaf(ga[e], rstd * (v[e] - mean), be[e]);
-          *reinterpret_cast<u32x2*>(ln_out + static_cast<int64_t>(r0 + r) * D + 4 * j) =
+          for (int e = 0; e < 4; ++e) o[e] = live ? fmaf(ga[e], rstd * (v[e] - mean), be[e]) : 0.f;
+          *reinterpret_cast<u32x2*>(out + static_cast<int64_t>(r0 + r) * D + 4 * j) =
               u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
         }
       }
@@ -287,7 +288,7 @@ hipError_t launch_tail(const BlockTailArgs& a, int rows, float eps, int num_cus,
   const int slabs = (rows + kTailRows - 1) / kTailRows;
   const int grid = slabs < num_cus ? slabs : num_cus;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(kTailThreads), kLds, st, a.ctx, a.x, a.wo, a.bo, a.g2, a.be2, a.w1,
-                     a.b1, a.w2, a.b2, a.out, rows, eps, a.row_mask, a.g1n, a.be1n, a.ln_out);
+                     a.b1, a.w2, a.b2, a.out, rows, eps, a.row_mask, a.final_g, a.final_b);
   return hipGetLastError();
 }
 
@@ -313,7 +314,7 @@ hipError_t block_tail_bf16(const BlockTailArgs& a, int64_t rows, int64_t d_model
   if (rows == 0) return hipSuccess;
   if (!block_tail_supported(d_model, ffn_dim) || rows >= (int64_t(1) << 31)) return hipErrorInvalidValue;
   // the kernel reads x and writes out through restrict pointers
-  if (a.out == a.x || (a.ln_out != nullptr && (a.ln_out == a.x || a.ln_out == a.out))) return hipErrorInvalidValue;
+  if (a.out == a.x) return hipErrorInvalidValue;
   const int r = static_cast<int>(rows);
   switch (d_model) {
     case 32: return launch_tail_f<32>(static_cast<int>(ffn_dim), a, r, eps, num_cus, stream);

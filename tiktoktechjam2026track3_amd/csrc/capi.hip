@@ -273,27 +273,56 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
     return ok();
   }
 
-  // Narrow models with up to 8192 tokens run the block tail (out_proj ..
-  // ffn_out, and the next layer's norm1) as one kernel, whose 16-byte loads
-  // need 16-byte aligned weights (all but the QKV projection's).
-  // (With more tokens the four launches win: the fused kernel's one workgroup
-  // per CU cannot hide its per-slab latency; measured on MI355X.)
-  bool tail_fused = enc::block_tail_supported(D, F) && T <= 8192 && no_split;
-  for (int64_t layer = 0; tail_fused && layer < num_layers; ++layer)
-    for (int idx = 0; idx < 12; ++idx)
-      tail_fused = tail_fused && (idx == 2 || idx == 3 || reinterpret_cast<uintptr_t>(W(layer, idx)) % 16 == 0);
+  // Narrow models otherwise run three launches a layer: norm1 with the QKV
+  // projection, the attention, and everything after it (the last layer's with
+  // the final norm).  Same 16-byte alignment.
+  bool narrow = enc::narrow_rows_supported(T, seq_len, D, H, F) && no_split &&
+                (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+  for (int64_t i = 0; narrow && i < 12 * num_layers + 2; ++i)
+    narrow = reinterpret_cast<uintptr_t>(weights[i]) % 16 == 0;
+  auto attention = exact ? enc::attention_fwd_bf16 : enc::flash_attention_fwd_bf16;
 
   const bf16_t* cur = static_cast<const bf16_t*>(x);
   hipError_t e = hipSuccess;
-  bool ln_ready = false;  // the fused tail already wrote this layer's norm1
   for (int64_t layer = 0; layer < num_layers; ++layer) {
     bf16_t* x_attn = (cur == xa) ? xb : xa;  // residual stream after attention
-    // norm1
-    if (!ln_ready) {
-      e = enc::layernorm_bf16(cur, W(layer, 0), W(layer, 1), ln, T, D, eps, nullptr, st);
-      if (e != hipSuccess) return fail_hip(e, "encoder norm1");
+    if (narrow) {
+      e = enc::narrow_qkv_bf16(cur, W(layer, 0), W(layer, 1), W(layer, 2), W(layer, 3), q, k, vt, batch, seq_len, D, H,
+                               eps, cus, st);
+      if (e != hipSuccess) return fail_hip(e, "encoder norm1 and qkv");
+      e = attention(q, k, vt, ctx, static_cast<int>(batch), static_cast<int>(H), static_cast<int>(seq_len),
+                    static_cast<int>(D / H), scale, causal != 0, kv_len, key_mask, st);
+      if (e != hipSuccess) return fail_hip(e, "encoder attention");
+      const bool last = layer + 1 == num_layers;
+      enc::BlockTailArgs ta;
+      ta.ctx = ctx;
+      ta.x = cur;
+      ta.wo = W(layer, 4);
+      ta.bo = W(layer, 5);
+      ta.g2 = W(layer, 6);
+      ta.be2 = W(layer, 7);
+      ta.w1 = W(layer, 8);
+      ta.b1 = W(layer, 9);
+      ta.w2 = W(layer, 10);
+      ta.b2 = W(layer, 11);
+      ta.out = last ? static_cast<bf16_t*>(out) : x_attn;
+      ta.row_mask = row_mask;
+      if (last && final_norm) {
+        ta.final_g = static_cast<const bf16_t*>(weights[12 * num_layers]);
+        ta.final_b = static_cast<const bf16_t*>(weights[12 * num_layers + 1]);
+      }
+      // (block_tail_bf16 reads x through a restrict pointer; a one-layer
+      // forward in place with a final norm is not refused)
+      const bool rows_tail = enc::narrow_tail_faster(T) || (ta.out == ta.x && final_norm);
+      e = rows_tail ? enc::narrow_tail_bf16(ta, T, D, F, eps, cus, st)
+                    : enc::block_tail_bf16(ta, T, D, F, eps, cus, st);
+      if (e != hipSuccess) return fail_hip(e, "encoder block tail");
+      cur = ta.out;
+      continue;
     }
-    ln_ready = false;
+    // norm1
+    e = enc::layernorm_bf16(cur, W(layer, 0), W(layer, 1), ln, T, D, eps, nullptr, st);
+    if (e != hipSuccess) return fail_hip(e, "encoder norm1");
     // packed QKV, head-major
     enc::GemmEpilogueArgs qa;
     qa.bias = W(layer, 3);
@@ -309,36 +338,9 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
     e = enc::gemm_bf16(ln, W(layer, 2), T, 3 * D, D, enc::kEpiQkvHeadMajor, qa, cus, st);
     if (e != hipSuccess) return fail_hip(e, "encoder qkv");
     // attention -> context [T, D]
-    auto attention = exact ? enc::attention_fwd_bf16 : enc::flash_attention_fwd_bf16;
     e = attention(q, k, vt, ctx, static_cast<int>(batch), static_cast<int>(H), static_cast<int>(seq_len),
                   static_cast<int>(D / H), scale, causal != 0, kv_len, key_mask, st);
     if (e != hipSuccess) return fail_hip(e, "encoder attention");
-    if (tail_fused) {
-      // out_proj .. ffn_out in one launch (narrow models), same arithmetic
-      enc::BlockTailArgs ta;
-      ta.ctx = ctx;
-      ta.x = cur;
-      ta.wo = W(layer, 4);
-      ta.bo = W(layer, 5);
-      ta.g2 = W(layer, 6);
-      ta.be2 = W(layer, 7);
-      ta.w1 = W(layer, 8);
-      ta.b1 = W(layer, 9);
-      ta.w2 = W(layer, 10);
-      ta.b2 = W(layer, 11);
-      ta.out = (!final_norm && layer == num_layers - 1) ? static_cast<bf16_t*>(out) : x_attn;
-      ta.row_mask = row_mask;
-      if (layer + 1 < num_layers) {  // the next layer's norm1 comes with the tail
-        ta.g1n = W(layer + 1, 0);
-        ta.be1n = W(layer + 1, 1);
-        ta.ln_out = ln;
-        ln_ready = true;
-      }
-      e = enc::block_tail_bf16(ta, T, D, F, eps, cus, st);
-      if (e != hipSuccess) return fail_hip(e, "encoder block tail");
-      cur = ta.out;
-      continue;
-    }
     // out_proj + residual; padded rows keep the residual (attention output is 0 there)
     enc::GemmEpilogueArgs oa;
     oa.bias = W(layer, 5);
@@ -360,7 +362,7 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
     if (e != hipSuccess) return fail_hip(e, std::string("encoder ") + stage);
     cur = x_next;
   }
-  if (!final_norm) return ok();  // out holds the last block's output
+  if (!final_norm || narrow) return ok();  // out holds the last block's output
   e = enc::layernorm_bf16(cur, static_cast<const bf16_t*>(weights[12 * num_layers]),
                           static_cast<const bf16_t*>(weights[12 * num_layers + 1]), static_cast<bf16_t*>(out), T, D,
                           eps, row_mask, st);

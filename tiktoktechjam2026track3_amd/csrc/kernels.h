@@ -126,17 +126,29 @@ struct BlockTailArgs {
   const bf16_t* b1 = nullptr;
   const bf16_t* w2 = nullptr;   // ffn_out weight [D, F] and bias [D]
   const bf16_t* b2 = nullptr;
-  bf16_t* out = nullptr;        // block output [T, D]; must not alias x (rejected)
+  bf16_t* out = nullptr;        // block output [T, D]; block_tail_bf16: must not alias x (rejected)
   const uint8_t* row_mask = nullptr;
-  // optional: the next layer's norm1 (weight, bias) applied to the block
-  // output, written to ln_out [T, D] (no row mask, as the separate launch)
-  const bf16_t* g1n = nullptr;
-  const bf16_t* be1n = nullptr;
-  bf16_t* ln_out = nullptr;
+  // optional: the final norm (weight, bias), written in the block output's
+  // place (rows masked out stay 0)
+  const bf16_t* final_g = nullptr;
+  const bf16_t* final_b = nullptr;
 };
 bool block_tail_supported(int64_t d_model, int64_t ffn_dim);
 hipError_t block_tail_bf16(const BlockTailArgs& args, int64_t rows, int64_t d_model, int64_t ffn_dim, float eps,
                            int num_cus, hipStream_t stream);
+
+// The row-wise halves of a narrow model's layer (d_model and ffn_dim of 32, 64
+// or 128), bitwise the separate launches: norm1 and the packed QKV projection
+// (head-major Q and K, V^T with its padding columns written), and the block
+// tail for many tokens.  All operands 16-byte aligned; the tail may run in place.
+bool narrow_rows_supported(int64_t rows, int64_t seq_len, int64_t d_model, int64_t heads, int64_t ffn_dim);
+hipError_t narrow_qkv_bf16(const bf16_t* x, const bf16_t* gamma, const bf16_t* beta, const bf16_t* w,
+                           const bf16_t* bias, bf16_t* q, bf16_t* k, bf16_t* v_t, int64_t batch, int64_t seq_len,
+                           int64_t d_model, int64_t heads, float eps, int cus, hipStream_t stream);
+// Whether the tail is the faster one, of it and block_tail_bf16.
+bool narrow_tail_faster(int64_t rows);
+hipError_t narrow_tail_bf16(const BlockTailArgs& args, int64_t rows, int64_t d_model, int64_t ffn_dim, float eps,
+                            int cus, hipStream_t stream);
 
 // Whole forward of a narrow model in one launch (per kNarrowMaxLayers layers):
 // d_model and ffn_dim of 32, 64 or 128, at most 128 tokens a sequence, the

@@ -229,7 +229,7 @@ __device__ __forceinline__ void head_attention(const bf16x8 (&qf)[HD < 32 ? 1 : 
 // The heads run in groups of kGC channels so that K and V^T of a group, the
 // two stages, the GELU table and two layers' vectors fit twice in a CU's LDS.
 // A stage is as long as that allows: each costs a barrier (32-row stages at
-// d_model 128: 14% slower over 10000 sequences).
+// d_model 128: 3.39 ms against 3.21 for four layers of 10000 sequences).
 template <int D, int HD>
 struct Narrow {
   static constexpr int kNB = D / 32;                         // 32-feature blocks (u32x4 per lane) of a row
@@ -280,7 +280,7 @@ __device__ __forceinline__ void block_product(const bf16_t* frags, int lane, con
 // What bounds it: VALU issue (rocprofv3 on 10000 sequences of 128 tokens, d_model
 // 128, head dim 32: 80% of the cycles, about 4700 instructions a wavefront and
 // layer, more than half of them the exact softmax); in a small batch the
-// latency of one workgroup, 15 us a layer at 32 channels a head.  16 tokens a
+// latency of one workgroup, 30 us a layer at 32 channels a head.  16 tokens a
 // wavefront leave 128 registers, four wavefronts per SIMD (two workgroups of 77
 // KiB per CU; one at head dim 128): 32 tokens a wavefront at two per SIMD ran
 // the four layers of that batch in 3.71 ms against 3.17 ms here, the launches
@@ -642,24 +642,25 @@ bool narrow_forward_supported(int64_t S, int64_t D, int64_t H, int64_t F) {
   return S >= 1 && S <= 128 && narrow(D) && narrow(F) && D % H == 0 && (hd == 8 || narrow(hd));
 }
 
-// Where one launch beats the launch sequence, measured on MI355X, two layers,
-// us (sequence / one launch).  The sequence's time hardly moves up to 8192
-// tokens (43 - 57 us); one launch's hardly moves up to 256 workgroups, and
-// grows with the heads, which a wavefront takes one after the other:
+// Where one launch beats three launches a layer (narrow_rows.hip), measured on
+// MI355X, two layers, us (three a layer / one).  The sequence's time hardly moves
+// up to 8192 tokens (below 50 the host's launches count, not the kernels); one
+// launch's hardly moves up to 256 workgroups, and grows with the heads, which a
+// wavefront takes one after the other:
 //   d_model 32 and 64, 32 channels a head and more: always (d 64, hd 32, 8 x 128
-//     tokens 46.3 / 32.7, 128 x 128 114.8 / 34.2; d 32, 8 x 128 37.7 / 20.8);
-//   d 128, hd 64 and 128: 8 x 48 50.6 / 45.8, but 8 x 128 49.1 / 51.0, 51.3 /
-//     55.3, 32 x 128 54.7 / 51.8;
-//   d 128, hd 32: 32 x 128 56.0 / 66.2, 64 x 128 73.9 / 66.7, 64 x 32 52.1 / 53.2,
-//     128 x 32 57.5 / 53.7;
-//   hd 8 at d 32: 8 x 128 37.4 / 39.2, 32 x 128 41.0 / 39.5, 8 x 48 37.6 / 30.4;
-//     at d 64: 64 x 128 63.8 / 71.5, 128 x 128 148.0 / 73.4, 64 x 32 49.7 / 46.7;
-//     at d 128: 128 x 128 153.3 / 147.3, 128 x 32 82.7 / 96.3, 256 x 32 134.1 / 97.5.
+//     tokens level, 64 x 128 44.6 / 32.0, 256 x 128 65.5 / 34.0);
+//   d 128, hd 64 and 128: 32 x 128 56.3 / 58.1, 55.8 / 61.1, 64 x 128 55.2 /
+//     51.7, 57.7 / 55.3, 256 x 32 58.0 / 46.5;
+//   d 128, hd 32: 64 x 128 57.1 / 66.0, 128 x 128 81.9 / 68.3, 128 x 32 55.7 /
+//     59.5, 256 x 32 65.0 / 53.6;
+//   hd 8 at d 32: 32 x 128 level, 64 x 128 44.4 / 37.9; at d 64: 128 x 128 60.8 /
+//     71.0, 256 x 128 93.4 / 74.4, 256 x 32 68.5 / 45.3; at d 128: 128 x 128 109 /
+//     144, 256 x 128 155 / 156, 128 x 32 76.1 / 103, 256 x 32 112 / 96.8.
 bool narrow_forward_faster(int64_t B, int64_t S, int64_t D, int64_t H) {
   const int64_t hd = D / H;
-  if (hd == 8) return D == 32 ? B >= 32 || S <= 64 : B >= (D == 64 ? 80 : 160);
+  if (hd == 8) return D == 32 ? B >= 32 || S <= 64 : B >= (D == 64 ? 176 : 240);
   if (D < 128) return true;
-  return hd == 32 ? B >= 64 : B >= 16 || S <= 64;
+  return B >= (hd == 32 ? 96 : 48);
 }
 
 hipError_t narrow_forward_bf16(const NarrowForward& f, hipStream_t st) {
