@@ -2,6 +2,11 @@
 //
 //   C[M, N] = epilogue(A[M, K] . W[N, K]^T + bias)
 //
+// The kernels of this file, by shape: the ring kernel (gemm_big_kernel, direct
+// loads to LDS; see pick_big_tile), the skinny kernel for few rows, the narrow
+// one for N or K that are no multiple of 64, and the register-staged kernel
+// described next for what is left.
+//
 // A (activations) and W (nn.Linear weight, [out, in]) are both K-contiguous,
 // so both tiles are staged in LDS the same way: [rows][BK + 8] bf16, the 8-element
 // pad (16 bytes) spreading the 16-byte MFMA operand reads of 32 consecutive rows

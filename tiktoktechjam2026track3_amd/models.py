@@ -69,8 +69,8 @@ def even_row_block(seq_len: int, limit: int) -> int:
 
 # Token count up to which the candidate captures a HIP graph (launch-bound shapes).
 GRAPH_MAX_TOKENS = 4096
-# The tile-packed weight copies are read only by the wide GEMM kernel, which
-# runs products of at least this many rows; smaller inputs leave them unmade.
+# The tile-packed weight copies are read only by the wide GEMM kernel's larger
+# tiles; inputs of fewer rows than this leave them unmade.
 PACK_MIN_ROWS = 1024
 
 
