@@ -187,6 +187,35 @@ def test_encoder_parity_narrow_rows(device, cfg, masking):
             assert result["passed"], result
 
 
+@pytest.mark.parametrize("masked", [False, True], ids=["all", "masked"])
+@pytest.mark.parametrize("d_model", [32, 64, 128, 512])
+def test_encoder_forward_without_layers(device, d_model, masked):
+    """A forward of no layers is the final norm of its input (masked rows 0),
+    through both entry points, at the widths of the narrow models and past
+    them: bit for bit torch's LayerNorm."""
+    g = torch.Generator(device=device).manual_seed(d_model)
+    x = torch.randn(3, 37, d_model, generator=g, device=device).bfloat16()
+    gamma = (1 + 0.1 * torch.randn(d_model, generator=g, device=device)).bfloat16()
+    beta = (0.1 * torch.randn(d_model, generator=g, device=device)).bfloat16()
+    ref = torch.nn.functional.layer_norm(x, (d_model,), gamma, beta, 1e-5)
+    mask = row_mask = None
+    if masked:
+        mask = torch.rand(3, 37, generator=g, device=device) < 0.6
+        row_mask = mask.view(torch.uint8)
+        ref = ref.masked_fill(~mask[..., None], 0)
+    table = torch.tensor([gamma.data_ptr(), beta.data_ptr()], dtype=torch.int64)
+    workspace = torch.empty(native.encoder_workspace_bytes(3, 37, d_model, 1, d_model), device=device,
+                            dtype=torch.uint8)
+    heads = d_model // 32
+    for allocating in (True, False):
+        out = torch.full_like(x, float("nan"))
+        if allocating:
+            native.encoder_forward(x, out, workspace, table, heads, d_model, 0, 1e-5, True, None, None, row_mask)
+        else:
+            native.encoder_forward_noalloc(x, out, table, heads, d_model, 0, 1e-5, True, None, None, row_mask)
+        assert torch.equal(ref, out)
+
+
 @pytest.mark.parametrize(
     "cfg",
     [TransformerConfig(1, 100, 256, 4, 512, 3, True), TransformerConfig(2, 64, 512, 8, 1024, 2, False),

@@ -276,7 +276,7 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
   // Narrow models otherwise run three launches a layer: norm1 with the QKV
   // projection, the attention, and everything after it (the last layer's with
   // the final norm).  Same 16-byte alignment.
-  bool narrow = enc::narrow_rows_supported(T, seq_len, D, H, F) && no_split &&
+  bool narrow = num_layers > 0 && enc::narrow_rows_supported(T, seq_len, D, H, F) && no_split &&
                 (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
   for (int64_t i = 0; narrow && i < 12 * num_layers + 2; ++i)
     narrow = reinterpret_cast<uintptr_t>(weights[i]) % 16 == 0;
@@ -362,7 +362,7 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
     if (e != hipSuccess) return fail_hip(e, std::string("encoder ") + stage);
     cur = x_next;
   }
-  if (!final_norm || narrow) return ok();  // out holds the last block's output
+  if (!final_norm || narrow) return ok();  // the last layer wrote out (without layers narrow is false)
   e = enc::layernorm_bf16(cur, static_cast<const bf16_t*>(weights[12 * num_layers]),
                           static_cast<const bf16_t*>(weights[12 * num_layers + 1]), static_cast<bf16_t*>(out), T, D,
                           eps, row_mask, st);
