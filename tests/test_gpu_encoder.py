@@ -187,6 +187,35 @@ def test_encoder_parity_narrow_rows(device, cfg, masking):
             assert result["passed"], result
 
 
+@pytest.mark.parametrize("seq_len", [17, 29, 99])
+@pytest.mark.parametrize("d_model,causal", [(32, False), (64, True)])
+def test_narrow_one_launch_ignores_values_past_the_sequence(device, d_model, causal, seq_len):
+    """Tokens past the sequence that share a 16-token block with real ones:
+    their value row must not reach the real tokens' context, whatever it is.
+    Here it overflows (norm1's bias times V's weights is 2^130) while every
+    real token's stays finite: x is +-1 with a zero sum and +1 in feature 0, so
+    norm1's weight and bias of +-2^100 cancel there to about 2^82."""
+    cfg = TransformerConfig(64, seq_len, d_model, d_model // 32, d_model, 1, causal)
+    sd, candidate = build_models(cfg, 57, device)
+    g = torch.Generator(device=device).manual_seed(seq_len)
+    weights = {name: value.clone() for name, value in sd.items()}
+    weights["layers.0.norm1.weight"][0] = -(2.0**100)
+    weights["layers.0.norm1.bias"][0] = 2.0**100
+    for name, value in (("q", 0.0), ("k", 0.0), ("v", 2.0**30)):
+        weights[f"layers.0.attention.{name}_proj.weight"][:, 0] = value
+    weights["layers.0.attention.out_proj.weight"] *= 2.0**-112
+    candidate.load_state_dict(weights)
+    order = torch.rand(64, seq_len, d_model - 1, generator=g, device=device).argsort(-1)
+    x = torch.ones(64, seq_len, d_model, device=device, dtype=torch.bfloat16)
+    x[..., 1:] = torch.where(order < d_model // 2, -1.0, 1.0)
+    mask = torch.ones(64, seq_len, device=device, dtype=torch.bool)
+    with torch.inference_mode():
+        out = candidate(x, mask)
+        ref = encoder_forward(weights, x, mask, causal, cfg.num_heads, 1)
+    assert torch.isfinite(ref.float()).all()
+    assert torch.equal(ref, out)
+
+
 @pytest.mark.parametrize("masked", [False, True], ids=["all", "masked"])
 @pytest.mark.parametrize("d_model", [32, 64, 128, 512])
 def test_encoder_forward_without_layers(device, d_model, masked):

@@ -316,8 +316,11 @@ __global__ void __launch_bounds__(kWaves * kWave, 4) narrow_forward_kernel(const
   if (blockIdx.x & 1) qb = nw - 1 - qb;
   const int seq = blockIdx.x * spb + in_group;
   const bool live = in_group < spb && seq < a.B;  // uniform per wavefront
-  const int s = 16 * qb + l16;
-  const bool valid = live && s < S;
+  // A lane past the sequence repeats its last token, in every step and in the
+  // output's store (the same bits to the same row): its value meets zero
+  // weights only, and one that is not finite would still reach the context, as
+  // zeros in the token's place would that run norm1's bias through each layer.
+  const int s = min(16 * qb + l16, S - 1);
   const int64_t row = static_cast<int64_t>(seq) * S + s;
 
   Keys keys;
@@ -343,13 +346,13 @@ __global__ void __launch_bounds__(kWaves * kWave, 4) narrow_forward_kernel(const
   keys.pv_blocks = keys.causal ? min(limit_blocks, (keys.q32 | 1) + 1) : limit_blocks;
   const bool attends = live && !(a.kv_len != nullptr && 16 * qb >= kv_limit);
   keys.zero_row = a.kv_len != nullptr && s >= kv_limit;
-  const bool keep = a.row_mask == nullptr || (valid && a.row_mask[row] != 0);
+  const bool keep = a.row_mask == nullptr || (live && a.row_mask[row] != 0);
 
   u32x4 x[kNB];
 #pragma unroll
   for (int c = 0; c < kNB; ++c) {
     x[c] = u32x4{0u, 0u, 0u, 0u};
-    if (valid) x[c] = load16(a.x + row * D + 32 * c + g8);
+    if (live) x[c] = load16(a.x + row * D + 32 * c + g8);
   }
   // The GELU table's ready flag: one reading for the workgroup, before any
   // table word is read (a clear flag selects the erf, the same bits).  V^T's
@@ -611,7 +614,7 @@ __global__ void __launch_bounds__(kWaves * kWave, 4) narrow_forward_kernel(const
 #pragma unroll
       for (int e = 0; e < 4; ++e) x[c][e] = keep ? y[c][e] : 0u;
   }
-  if (valid) {
+  if (live) {
 #pragma unroll
     for (int c = 0; c < kNB; ++c) *reinterpret_cast<u32x4*>(a.out + row * D + 32 * c + g8) = x[c];
   }
