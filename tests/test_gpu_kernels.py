@@ -283,12 +283,16 @@ def test_linear_ring_tiles_bitwise(device, m, n, k, packed):
 @pytest.mark.parametrize(
     "b,s,d,h",
     [(64, 125, 1024, 4), (3, 777, 1024, 16), (300, 7, 1024, 16), (2100, 1, 512, 8), (1, 2049, 512, 8), (5, 129, 576, 9),
-     (90, 23, 1024, 128), (41, 50, 2048, 16)],
+     (90, 23, 1024, 128), (41, 50, 2048, 16), (2100, 1, 256, 4), (6001, 1, 256, 4), (9000, 1, 1024, 16),
+     (3000, 2, 256, 4), (2731, 3, 512, 8), (260, 8, 256, 4), (750, 8, 512, 8), (1125, 8, 1024, 16), (130, 16, 512, 8),
+     (375, 24, 1024, 16), (70, 56, 256, 4), (64, 64, 512, 8)],
 )
 def test_qkv_ragged_sequences_bitwise(device, b, s, d, h):
-    """The ring kernel's V^T of sequences that are no whole number of 8-row
-    groups, on every tile: groups cut by a tile's edge, sequences shorter than
-    a group and than a tile's stride, many sequences a tile, one a grid."""
+    """The ring kernel's V^T of short sequences and of those that are no whole
+    number of 8-row groups, on every tile: groups cut by a tile's edge,
+    sequences of one token (full tiles and a partial last one), shorter than a
+    group and than a tile's stride (whole groups too), many sequences a tile,
+    one a grid."""
     g = torch.Generator(device=device).manual_seed(b + s + d)
     x = torch.randn(b, s, d, generator=g, device=device).bfloat16()
     w = (torch.randn(3 * d, d, generator=g, device=device) / math.sqrt(d)).bfloat16()

@@ -1052,97 +1052,134 @@ gemm_big_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int 
         }
       }
     }
-    // V^T on full tiles: two adjacent channels (one head: hd is even), 8
-    // consecutive rows (sequence positions).  Thread t owns channels
-    // 2 (t % (BN/2)) and +1, and row groups t / (BN/2), + kVStep2, ... of 8
-    // rows each: one 4-byte LDS read per row gives both channels' values,
-    // and byte permutes split them into one 16-byte V^T store per channel
-    // (half the LDS reads of one channel per thread).  Element offset of
-    // (b, s): b H hd ld + (h hd + d) ld + s.
+    // V^T: two adjacent channels (one head: hd is even) at 8 consecutive
+    // positions of a sequence.  Thread t owns channels 2 (t % (BN/2)) and +1,
+    // and groups t / (BN/2), + kVStep2, ... of 8 positions each: one 4-byte LDS
+    // read per row gives both channels' values, and byte permutes split them
+    // into one 16-byte V^T store per channel (half the LDS reads of one channel
+    // per thread).  Element offset of (b, s): b H hd ld + (h hd + d) ld + s.
+    auto store_pair8 = [](bf16_t* dst, int ld, const uint32_t (&w)[8]) __attribute__((always_inline)) {
+      u32x4 lo, hi;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = __builtin_amdgcn_perm(w[2 * e + 1], w[2 * e], 0x05040100u);  // rows 2e, 2e+1 of channel cp
+        hi[e] = __builtin_amdgcn_perm(w[2 * e + 1], w[2 * e], 0x07060302u);  // ... of channel cp + 1
+      }
+      *reinterpret_cast<u32x4*>(dst) = lo;
+      *reinterpret_cast<u32x4*>(dst + ld) = hi;
+    };
     constexpr int kVPairs = BN / 2;
     static_assert(kThreads % kVPairs == 0 && BM % (8 * (kThreads / kVPairs)) == 0, "channel pairs per thread");
     constexpr int kVStep2 = kThreads / kVPairs;
     const int cp = 2 * (tid % kVPairs);
-    const bool v_fast = full && (S & 7) == 0 && (ep.ld_vt & 7) == 0 && 8 * kVStep2 <= S;
-    if (v_fast && (n0 + cp) / D == 2) {
-      const int h = (n0 + cp - 2 * D) / hd;
-      const int d = (n0 + cp - 2 * D) - h * hd;
-      bf16_t* vrow = ep.v_t + (static_cast<int64_t>(h) * hd + d) * ep.ld_vt;
-      const int64_t batch_stride = static_cast<int64_t>(ep.num_heads) * hd * ep.ld_vt;
-      int b, s;
-      locate(m0 + (tid / kVPairs) * 8, b, s);
-      int64_t off = b * batch_stride + s;
+    // On full tiles of whole groups the groups are 8 rows of the tile, and the
+    // position is carried along (one wrap per step at most).
+    const bool v_groups = full && (S & 7) == 0 && (ep.ld_vt & 7) == 0;
+    if (S == 1 || (v_groups && S < 8 * kVStep2)) {
+      // Sequences shorter than a step: V^T's rows are so short that those of
+      // adjacent channels share a line, so a thread takes one channel (thread t
+      // channel t % BN, groups t / BN, + kVStep, ...) and neighbours store next
+      // to each other (6000x768x256, S = 1, 35.4 us by the last branch's groups
+      // -> 12.9; 2000x1536x512, S = 8, 22.7 -> 20.5; 6000x6144x2048, S = 16, 161
+      // by pairs -> 152).
+      constexpr int kVStep = kThreads / BN;
+      const int cl = tid % BN;
+      if ((n0 + cl) / D == 2) {
+        const int h = (n0 + cl - 2 * D) / hd;
+        const int d = (n0 + cl - 2 * D) - h * hd;
+        bf16_t* vrow = ep.v_t + (static_cast<int64_t>(h) * hd + d) * ep.ld_vt;
+        const int64_t batch_stride = static_cast<int64_t>(ep.num_heads) * hd * ep.ld_vt;
+        const int rows = min(BM, M - m0);
+        const int step_seqs = 8 * kVStep / S;
+        const int step_pos = 8 * kVStep - step_seqs * S;
+        int b, s;
+        locate(m0 + (tid / BN) * 8, b, s);
+        int64_t off = b * batch_stride + s;
+        for (int r8 = (tid / BN) * 8; r8 < rows; r8 += 8 * kVStep) {
+          uint32_t w[8];
 #pragma unroll
-      for (int it = 0; it < BM / (8 * kVStep2); ++it) {
-        const int r8 = (tid / kVPairs + it * kVStep2) * 8;
-        uint32_t w[8];  // row r8 + e: channel cp in the low half, cp + 1 in the high half
+          for (int e = 0; e < 8; ++e) w[e] = sc[(r8 + e) * T::kLdc + cl];
+          if (S == 1) {  // one value and seven padding columns, which keep the store whole
 #pragma unroll
-        for (int e = 0; e < 8; ++e) w[e] = *reinterpret_cast<const uint32_t*>(sc + (r8 + e) * T::kLdc + cp);
-        u32x4 lo, hi;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          lo[e] = __builtin_amdgcn_perm(w[2 * e + 1], w[2 * e], 0x05040100u);  // rows 2e, 2e+1 of channel cp
-          hi[e] = __builtin_amdgcn_perm(w[2 * e + 1], w[2 * e], 0x07060302u);  // ... of channel cp + 1
+            for (int e = 0; e < 8; ++e)
+              if (r8 + e < rows) *reinterpret_cast<u32x4*>(vrow + off + e * batch_stride) = u32x4{w[e], 0u, 0u, 0u};
+          } else {
+            *reinterpret_cast<u32x4*>(vrow + off) =
+                u32x4{w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16)};
+          }
+          s += step_pos;
+          off += step_seqs * batch_stride + step_pos;
+          const bool wrap = s >= S;
+          s = wrap ? s - S : s;
+          off = wrap ? off + batch_stride - S : off;
         }
-        *reinterpret_cast<u32x4*>(vrow + off) = lo;
-        *reinterpret_cast<u32x4*>(vrow + ep.ld_vt + off) = hi;
-        s += 8 * kVStep2;
-        off += 8 * kVStep2;
-        const bool wrap = s >= S;
-        s = wrap ? s - S : s;
-        off = wrap ? off + batch_stride - S : off;
       }
-    }
-    // V^T otherwise (a partial tile, or sequences that are no whole number of
-    // 8-row groups): the groups follow the sequences instead of the tile's
-    // rows, eight positions from a multiple of 8 on, so that a group is one
-    // 16-byte store again.  Group v covers positions 8 (v % G) .. of sequence
-    // v / G, G = ld_vt / 8; a sequence's last one may run into its padding
-    // columns, which nobody reads; only the groups that the tile's first and
-    // last row cut are stored by element.  (Every element by itself, with a
-    // division each, as groups of tile rows have to be: 8000x3072x1024, S = 125,
-    // 122 us against 64.5.)
-    if (!v_fast && (n0 + cp) / D == 2) {
+    } else if ((n0 + cp) / D == 2) {
       const int h = (n0 + cp - 2 * D) / hd;
       const int d = (n0 + cp - 2 * D) - h * hd;
       bf16_t* vrow = ep.v_t + (static_cast<int64_t>(h) * hd + d) * ep.ld_vt;
       const int64_t batch_stride = static_cast<int64_t>(ep.num_heads) * hd * ep.ld_vt;
-      const int groups = ep.ld_vt / 8;
-      const int last = min(m0 + BM, M) - 1;
-      int b, s, b_end, s_end;
-      locate(m0, b, s);
-      locate(last, b_end, s_end);
-      int sg = s / 8 + tid / kVPairs;  // this thread's first group of sequence b
-      for (;;) {
-        while (sg >= groups) {
-          sg -= groups;
-          ++b;
-        }
-        if (b > b_end || (b == b_end && sg > s_end / 8)) break;
-        const int row0 = b * S + 8 * sg - m0;              // tile row of the group's first position
-        const int rows = min(8, S - 8 * sg);
-        bf16_t* dst = vrow + b * batch_stride + 8 * sg;
-        if (row0 >= 0 && row0 + rows - 1 + m0 <= last) {
-          uint32_t w[8];  // position e: channel cp in the low half, cp + 1 in the high half
+      if (v_groups) {
+        int b, s;
+        locate(m0 + (tid / kVPairs) * 8, b, s);
+        int64_t off = b * batch_stride + s;
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            w[e] = *reinterpret_cast<const uint32_t*>(sc + (row0 + min(e, rows - 1)) * T::kLdc + cp);
-          u32x4 lo, hi;
+        for (int it = 0; it < BM / (8 * kVStep2); ++it) {
+          const int r8 = (tid / kVPairs + it * kVStep2) * 8;
+          uint32_t w[8];  // row r8 + e: channel cp in the low half, cp + 1 in the high half
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            lo[e] = __builtin_amdgcn_perm(w[2 * e + 1], w[2 * e], 0x05040100u);
-            hi[e] = __builtin_amdgcn_perm(w[2 * e + 1], w[2 * e], 0x07060302u);
-          }
-          *reinterpret_cast<u32x4*>(dst) = lo;
-          *reinterpret_cast<u32x4*>(dst + ep.ld_vt) = hi;
-        } else {
-          for (int e = 0; e < rows; ++e) {
-            if (row0 + e < 0 || row0 + e + m0 > last) continue;
-            dst[e] = sc[(row0 + e) * T::kLdc + cp];
-            dst[ep.ld_vt + e] = sc[(row0 + e) * T::kLdc + cp + 1];
-          }
+          for (int e = 0; e < 8; ++e) w[e] = *reinterpret_cast<const uint32_t*>(sc + (r8 + e) * T::kLdc + cp);
+          store_pair8(vrow + off, ep.ld_vt, w);
+          s += 8 * kVStep2;
+          off += 8 * kVStep2;
+          const bool wrap = s >= S;
+          s = wrap ? s - S : s;
+          off = wrap ? off + batch_stride - S : off;
         }
-        sg += kVStep2;
+      } else {
+        // A partial tile, or sequences that are no whole number of groups: the
+        // groups follow the sequences instead of the tile's rows, eight positions
+        // from a multiple of 8 on, so that a group is one 16-byte store again.
+        // Group v covers positions 8 (v % G) .. of sequence v / G, G = ld_vt / 8;
+        // a sequence's last one may run into its padding columns, which nobody
+        // reads; only the groups that the tile's first and last row cut are stored
+        // by element.  (Every element by itself, with a division each, as groups of
+        // tile rows have to be: 8000x3072x1024, S = 125, 122 us against 64.5.)  A
+        // step is step_seqs sequences and step_groups groups (counted down one
+        // sequence at a time it cost 6000x1536x512, S = 8, 22.7 us against 20.0).
+        const int groups = ep.ld_vt / 8;
+        const int step_seqs = kVStep2 < groups ? 0 : kVStep2 / groups;
+        const int step_groups = kVStep2 - step_seqs * groups;
+        const int last = min(m0 + BM, M) - 1;
+        int b, s, b_end, s_end;
+        locate(m0, b, s);
+        locate(last, b_end, s_end);
+        int sg = s / 8 + tid / kVPairs;  // this thread's first group of sequence b
+        b += sg / groups;
+        sg %= groups;
+        while (b < b_end || (b == b_end && sg <= s_end / 8)) {
+          const int row0 = b * S + 8 * sg - m0;              // tile row of the group's first position
+          const int rows = min(8, S - 8 * sg);
+          bf16_t* dst = vrow + b * batch_stride + 8 * sg;
+          if (row0 >= 0 && row0 + rows - 1 + m0 <= last) {
+            uint32_t w[8];  // position e: channel cp in the low half, cp + 1 in the high half
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              w[e] = *reinterpret_cast<const uint32_t*>(sc + (row0 + min(e, rows - 1)) * T::kLdc + cp);
+            store_pair8(dst, ep.ld_vt, w);
+          } else {
+            for (int e = 0; e < rows; ++e) {
+              if (row0 + e < 0 || row0 + e + m0 > last) continue;
+              dst[e] = sc[(row0 + e) * T::kLdc + cp];
+              dst[ep.ld_vt + e] = sc[(row0 + e) * T::kLdc + cp + 1];
+            }
+          }
+          b += step_seqs;
+          sg += step_groups;
+          const bool wrap = sg >= groups;
+          sg = wrap ? sg - groups : sg;
+          b = wrap ? b + 1 : b;
+        }
       }
     }
   }
@@ -1777,7 +1814,7 @@ hipError_t launch_tail_split(const bf16_t* A, const bf16_t* W, int M, int N, int
 // should run: the operands must be 16-byte aligned (16-byte loads per lane),
 // the residual / outputs too (16-byte epilogue stores).
 int pick_big_tile(int64_t M, int64_t N, const bf16_t* A, const bf16_t* W, const GemmEpilogueArgs& ep,
-                  bool ep_overlaps, int num_cus) {
+                  int epi, int num_cus) {
   auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (!al(A) || !al(W) || !al(ep.out) || !al(ep.residual) || !al(ep.q) || !al(ep.k) || !al(ep.v_t) ||
       !al(ep.w_packed) || reinterpret_cast<uintptr_t>(ep.bias) % 8 != 0)  // 8-byte bias loads
@@ -1799,15 +1836,16 @@ int pick_big_tile(int64_t M, int64_t N, const bf16_t* A, const bf16_t* W, const 
   // 8000x2048x2048 81.5 vs 89.5).  The residual epilogues run as fast or faster
   // on the 256x256 tiles (32768x1024x1024 plain weight: 73.5 vs 83.2 us;
   // 409600x1024x1024 packed: 932 vs 1007 us).
-  if (ep_overlaps && tiles(256, 128) >= 2 * num_cus) return 256129;
-  if (ep_overlaps && tiles(128, 128) > num_cus) return 128129;
+  if (epi == kEpiBiasGelu) {
+    if (tiles(256, 128) >= 2 * num_cus) return 256129;
+    if (tiles(128, 128) > num_cus) return 128129;
+  }
   // Whole rounds of tiles over the CUs times the tile's work, over its
   // efficiency: one full round at K = 1024 takes 34.5, 20.9 and 11.7 us on
   // 256x256, 256x128 and 128x128 tiles, and several rounds of 128x128 tiles
   // slow each other (9000x2048x2048: 5 rounds 88.8 us, 3 of 256x128 84.9).
-  // (2331x2048x2048, where 128x128 tiles need
-  // a second round: 33.5 -> 25.5 us on 256x128; 1500x4096x1024 20.4 -> 17.3;
-  // QKV 2048x3072x1024 24.2 -> 20.8.)
+  // (2331x2048x2048, where 128x128 tiles need a second round: 33.5 -> 25.5 us on
+  // 256x128; 1500x4096x1024 20.4 -> 17.3; QKV 2048x3072x1024 24.2 -> 20.8.)
   auto cost = [&](int bm, int bn, double eff) {
     const int64_t rounds = (tiles(bm, bn) + num_cus - 1) / num_cus;
     return static_cast<double>(rounds) * bm * bn / eff;
@@ -1815,7 +1853,12 @@ int pick_big_tile(int64_t M, int64_t N, const bf16_t* A, const bf16_t* W, const 
   const double c256 = N % 256 == 0 ? cost(256, 256, 1.0) : 1e30;
   const double c128 = cost(256, 128, 0.83), c64 = cost(128, 128, 0.68);
   if (c256 <= c128 && c256 <= c64) return 256256;
-  return c128 <= c64 ? 256128 : 128128;
+  if (c128 > c64) return 128128;
+  // V^T of sequences of one or two tokens is mostly padding, up to eight times
+  // its values, and written by a third of the tiles: a long epilogue again
+  // (S = 2: 6000x768x256 18.9 -> 13.6 us, 3000x1536x512 21.6 -> 17.2).
+  if (epi == kEpiQkvHeadMajor && ep.seq_len <= 2) return 128129;
+  return 256128;
 }
 
 }  // namespace
@@ -1939,12 +1982,11 @@ hipError_t gemm_bf16_plain(const bf16_t* A, const bf16_t* W, int64_t M, int64_t 
   if (split == 4 && chunk == 32) return launch_split<4, 32>(A, W, m, n, k, epi, ep, stream);
   if (split == 4 && chunk == 64) return launch_split<4, 64>(A, W, m, n, k, epi, ep, stream);
   if (split == 2 && chunk == 128) return launch_split<2, 128>(A, W, m, n, k, epi, ep, stream);
-  const bool ep_overlaps = epi == kEpiBiasGelu;
   // The large-tile head-major epilogue stores 8 channels of one head at a
   // time (Q, K) and channel pairs (V^T, in 16-byte pieces of its rows):
   // head_dim and ld_vt must be multiples of 8.
   const bool big_ok = epi != kEpiQkvHeadMajor || (ep.head_dim % 8 == 0 && ep.ld_vt % 8 == 0);
-  switch (big_ok ? pick_big_tile(M, N, A, W, ep, ep_overlaps, num_cus) : 0) {
+  switch (big_ok ? pick_big_tile(M, N, A, W, ep, epi, num_cus) : 0) {
     case 256129: return launch_big<256, 128, 32, 3, 2>(A, W, m, n, k, epi, ep, stream);
     // 256x256 tiles: from the plain nn.Linear weight, 64-deep K blocks in two
     // stages (32768x3072x1024: 190 vs 201 us); from the tile-packed copy,
