@@ -1813,7 +1813,7 @@ hipError_t launch_tail_split(const bf16_t* A, const bf16_t* W, int M, int N, int
 // Tile of the ring kernel for this shape, or 0 when the register-staged kernel
 // should run: the operands must be 16-byte aligned (16-byte loads per lane),
 // the residual / outputs too (16-byte epilogue stores).
-int pick_big_tile(int64_t M, int64_t N, const bf16_t* A, const bf16_t* W, const GemmEpilogueArgs& ep,
+int pick_big_tile(int64_t M, int64_t N, int64_t K, const bf16_t* A, const bf16_t* W, const GemmEpilogueArgs& ep,
                   int epi, int num_cus) {
   auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (!al(A) || !al(W) || !al(ep.out) || !al(ep.residual) || !al(ep.q) || !al(ep.k) || !al(ep.v_t) ||
@@ -1832,26 +1832,32 @@ int pick_big_tile(int64_t M, int64_t N, const bf16_t* A, const bf16_t* W, const 
   // MFMA loop.  It pays where the epilogue is long against the K loop, the
   // GELU: 256x128 tiles when there are two for every CU (32768x4096x1024: 314
   // vs 366 us on 256x256 tiles), else 128x128 tiles when there is more than
-  // one (2331x4096x1024: 36.8 vs 45.1 us, 1500x4096x1024 22.2 vs 28.2,
-  // 8000x2048x2048 81.5 vs 89.5).  The residual epilogues run as fast or faster
-  // on the 256x256 tiles (32768x1024x1024 plain weight: 73.5 vs 83.2 us;
+  // one and the K loop is short (us, 128x128 / the choice by rounds below:
+  // 2331x4096x1024 36.8 / 45.1, 5788x2048x256 21.6 / 28.3, 3000x4096x2048 65.0 /
+  // 66.1; past three a CU the K loops slow each other, 9057x1536x2048 71.4 /
+  // 67.2, and with a long K from the first on, 3017x1536x4096 57.9 / 51.1,
+  // 5099x3072x4096 130 / 116).  The residual epilogues run as fast or faster on
+  // the 256x256 tiles (32768x1024x1024 plain weight: 73.5 vs 83.2 us;
   // 409600x1024x1024 packed: 932 vs 1007 us).
   if (epi == kEpiBiasGelu) {
     if (tiles(256, 128) >= 2 * num_cus) return 256129;
-    if (tiles(128, 128) > num_cus) return 128129;
+    if (tiles(128, 128) > num_cus && (K <= 1024 || (K <= 2048 && tiles(128, 128) <= 3 * num_cus))) return 128129;
   }
   // Whole rounds of tiles over the CUs times the tile's work, over its
   // efficiency: one full round at K = 1024 takes 34.5, 20.9 and 11.7 us on
   // 256x256, 256x128 and 128x128 tiles, and several rounds of 128x128 tiles
   // slow each other (9000x2048x2048: 5 rounds 88.8 us, 3 of 256x128 84.9).
   // (2331x2048x2048, where 128x128 tiles need a second round: 33.5 -> 25.5 us on
-  // 256x128; 1500x4096x1024 20.4 -> 17.3; QKV 2048x3072x1024 24.2 -> 20.8.)
+  // 256x128; 1500x4096x1024 20.4 -> 17.3; QKV 2048x3072x1024 24.2 -> 20.8.  Over
+  // 300 products of K 256 to 4096 the choice is the fastest tile's time within
+  // 1.4% on average, the same for 0.86 to 0.90; 6000x6144x2048: 158 us on 256x128,
+  // 163 to 167 on 256x256, which 0.83 would take.)
   auto cost = [&](int bm, int bn, double eff) {
     const int64_t rounds = (tiles(bm, bn) + num_cus - 1) / num_cus;
     return static_cast<double>(rounds) * bm * bn / eff;
   };
   const double c256 = N % 256 == 0 ? cost(256, 256, 1.0) : 1e30;
-  const double c128 = cost(256, 128, 0.83), c64 = cost(128, 128, 0.68);
+  const double c128 = cost(256, 128, 0.88), c64 = cost(128, 128, 0.68);
   if (c256 <= c128 && c256 <= c64) return 256256;
   if (c128 > c64) return 128128;
   // V^T of sequences of one or two tokens is mostly padding, up to eight times
@@ -1986,7 +1992,7 @@ hipError_t gemm_bf16_plain(const bf16_t* A, const bf16_t* W, int64_t M, int64_t 
   // time (Q, K) and channel pairs (V^T, in 16-byte pieces of its rows):
   // head_dim and ld_vt must be multiples of 8.
   const bool big_ok = epi != kEpiQkvHeadMajor || (ep.head_dim % 8 == 0 && ep.ld_vt % 8 == 0);
-  switch (big_ok ? pick_big_tile(M, N, A, W, ep, epi, num_cus) : 0) {
+  switch (big_ok ? pick_big_tile(M, N, K, A, W, ep, epi, num_cus) : 0) {
     case 256129: return launch_big<256, 128, 32, 3, 2>(A, W, m, n, k, epi, ep, stream);
     // 256x256 tiles: from the plain nn.Linear weight, 64-deep K blocks in two
     // stages (32768x3072x1024: 190 vs 201 us); from the tile-packed copy,
