@@ -1035,7 +1035,10 @@ hipError_t dispatch_order(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf
   // registers, in every sweep, which one wavefront does too slowly from the
   // head dim on that the rule names (128 1 x 8 x 200 24.7 / 20.3, 1 x 8 x 1000
   // 78.6 / 72.0; 64 1 x 8 x 300 23.5 / 21.3; 32 1 x 8 x 200 15.2 / 14.3, but 1
-  // x 8 x 1000 48.0 / 50.5).
+  // x 8 x 1000 48.0 / 50.5).  That holds for a prefix mask too, whose lengths
+  // the host does not know: a batch is padded to its longest sequence, which
+  // reaches the last tile (64 8 x 4 x 300 25.2 / 21.5; one whose sequences all
+  // end before it would run 16.8 / 19.4).
   // Head dim 256 streams its rows by four wavefronts however small the grid:
   // its ring takes 128 KiB, and one wavefront's load offsets for whole tiles
   // leave the registers (480 bytes of scratch).  4 x 4 heads of 1024 causal
@@ -1082,11 +1085,33 @@ hipError_t dispatch_order(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf
   }
   // Head dims 8 and 32: the softmax's per-score operations are all there is,
   // and four wavefronts per SIMD with the half-tile sweeps hide more of their
-  // latency than two: 64 x 4 heads of 32, 1024 causal keys 175.6 -> 168.7 us,
-  // prefix 777 95.4 -> 92.7, 200 x 4 x 300 118.9 -> 116.9, byte masks level;
-  // 64 x 16 heads of 8, 1024 causal keys 557 -> 532.
-  if constexpr (HD <= 32)
-    return launch_attn<HD, 4, CAUSAL, MASK, POW2, false, 0, 4>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
+  // latency than two, once there are workgroups to fill them: 1024 are resident
+  // at a time then, 512 with two.  Between the two, causal rows have their long
+  // and short workgroups side by side all through, where two wavefronts per
+  // SIMD start the short ones as the long ones end; prefix masks, whose rows
+  // differ too, need more rounds to even out.  Times of four over two, 64 x 4
+  // heads' worth of forms at 512 to 3072 workgroups, S 257 to 2048:
+  //   head dim 8: no mask 0.94 - 1.00; causal 0.91 - 1.00, but 1.00 - 1.03 from
+  //     900 to 1300 workgroups past 640 keys; prefix 0.95 - 1.01 from 1200 on
+  //     (1.21 at 896); causal prefix 0.92 - 1.02 to 800 workgroups and from 2560
+  //     on (1600 to 512 keys), 0.94 - 1.12 between; bytes 1.01 - 1.03, causal
+  //     0.86 - 1.00 from 1400 on.
+  //   head dim 32: no mask 0.97 - 1.01 from 1024 on (to 1.03 below); causal 0.91 -
+  //     1.01, 1.01 - 1.06 from 900 to 1300 past 640 keys; prefix 0.95 - 1.04 from
+  //     1200 on (1.13 at 896), causal prefix 0.93 - 1.02 from 2560 on (1600), to
+  //     1.14 below; bytes 0.98 - 1.07.
+  if constexpr (HD <= 32 && (MASK != kMaskBytes || (HD == 8 && CAUSAL))) {
+    const bool few = groups128 <= 800 && MASK != kMaskBytes && (HD == 8 || (CAUSAL && MASK == kMaskNone));
+    int64_t from;
+    if (MASK == kMaskPrefix)
+      from = !CAUSAL ? 1200 : S <= 512 ? 1600 : 2560;
+    else if (CAUSAL)
+      from = MASK == kMaskNone && S <= 640 ? 0 : 1400;
+    else
+      from = HD == 8 ? 0 : 1024;
+    if (few || groups128 >= from)
+      return launch_attn<HD, 4, CAUSAL, MASK, POW2, false, 0, 4>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
+  }
   return launch_attn<HD, 4, CAUSAL, MASK, POW2, false>(q, k, vt, ctx, B, H, S, scale, kv_len, key_mask, st);
 }
 
