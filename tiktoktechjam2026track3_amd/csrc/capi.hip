@@ -273,9 +273,8 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
     return ok();
   }
 
-  // Narrow models otherwise run three launches a layer: norm1 with the QKV
-  // projection, the attention, and everything after it (the last layer's with
-  // the final norm).  Same 16-byte alignment.
+  // Narrow models otherwise run three launches a layer (four where norm1 and the
+  // QKV projection are faster apart).  Same 16-byte alignment.
   bool narrow = num_layers > 0 && enc::narrow_rows_supported(T, seq_len, D, H, F) && no_split &&
                 (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
   for (int64_t i = 0; narrow && i < 12 * num_layers + 2; ++i)
@@ -286,13 +285,35 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
   hipError_t e = hipSuccess;
   for (int64_t layer = 0; layer < num_layers; ++layer) {
     bf16_t* x_attn = (cur == xa) ? xb : xa;  // residual stream after attention
-    if (narrow) {
+    if (narrow && enc::narrow_qkv_faster(T, seq_len, D)) {
       e = enc::narrow_qkv_bf16(cur, W(layer, 0), W(layer, 1), W(layer, 2), W(layer, 3), q, k, vt, batch, seq_len, D, H,
                                eps, cus, st);
       if (e != hipSuccess) return fail_hip(e, "encoder norm1 and qkv");
-      e = attention(q, k, vt, ctx, static_cast<int>(batch), static_cast<int>(H), static_cast<int>(seq_len),
-                    static_cast<int>(D / H), scale, causal != 0, kv_len, key_mask, st);
-      if (e != hipSuccess) return fail_hip(e, "encoder attention");
+    } else {
+      // norm1
+      e = enc::layernorm_bf16(cur, W(layer, 0), W(layer, 1), ln, T, D, eps, nullptr, st);
+      if (e != hipSuccess) return fail_hip(e, "encoder norm1");
+      // packed QKV, head-major
+      enc::GemmEpilogueArgs qa;
+      qa.bias = W(layer, 3);
+      qa.q = q;
+      qa.k = k;
+      qa.v_t = vt;
+      qa.seq_len = static_cast<int>(seq_len);
+      qa.num_heads = static_cast<int>(H);
+      qa.head_dim = static_cast<int>(D / H);
+      qa.d_model = static_cast<int>(D);
+      qa.ld_vt = static_cast<int>(enc::vt_stride(seq_len));
+      use_packed(qa, layer, 0, 3 * D, D);
+      e = enc::gemm_bf16(ln, W(layer, 2), T, 3 * D, D, enc::kEpiQkvHeadMajor, qa, cus, st);
+      if (e != hipSuccess) return fail_hip(e, "encoder qkv");
+    }
+    // attention -> context [T, D]
+    e = attention(q, k, vt, ctx, static_cast<int>(batch), static_cast<int>(H), static_cast<int>(seq_len),
+                  static_cast<int>(D / H), scale, causal != 0, kv_len, key_mask, st);
+    if (e != hipSuccess) return fail_hip(e, "encoder attention");
+    if (narrow) {
+      // everything after it (the last layer's with the final norm)
       const bool last = layer + 1 == num_layers;
       enc::BlockTailArgs ta;
       ta.ctx = ctx;
@@ -320,27 +341,6 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
       cur = ta.out;
       continue;
     }
-    // norm1
-    e = enc::layernorm_bf16(cur, W(layer, 0), W(layer, 1), ln, T, D, eps, nullptr, st);
-    if (e != hipSuccess) return fail_hip(e, "encoder norm1");
-    // packed QKV, head-major
-    enc::GemmEpilogueArgs qa;
-    qa.bias = W(layer, 3);
-    qa.q = q;
-    qa.k = k;
-    qa.v_t = vt;
-    qa.seq_len = static_cast<int>(seq_len);
-    qa.num_heads = static_cast<int>(H);
-    qa.head_dim = static_cast<int>(D / H);
-    qa.d_model = static_cast<int>(D);
-    qa.ld_vt = static_cast<int>(enc::vt_stride(seq_len));
-    use_packed(qa, layer, 0, 3 * D, D);
-    e = enc::gemm_bf16(ln, W(layer, 2), T, 3 * D, D, enc::kEpiQkvHeadMajor, qa, cus, st);
-    if (e != hipSuccess) return fail_hip(e, "encoder qkv");
-    // attention -> context [T, D]
-    e = attention(q, k, vt, ctx, static_cast<int>(batch), static_cast<int>(H), static_cast<int>(seq_len),
-                  static_cast<int>(D / H), scale, causal != 0, kv_len, key_mask, st);
-    if (e != hipSuccess) return fail_hip(e, "encoder attention");
     // out_proj + residual; padded rows keep the residual (attention output is 0 there)
     enc::GemmEpilogueArgs oa;
     oa.bias = W(layer, 5);

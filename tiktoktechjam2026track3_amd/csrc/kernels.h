@@ -142,6 +142,8 @@ hipError_t block_tail_bf16(const BlockTailArgs& args, int64_t rows, int64_t d_mo
 // (head-major Q and K, V^T with its padding columns written), and the block
 // tail for many tokens.  All operands 16-byte aligned; the tail may run in place.
 bool narrow_rows_supported(int64_t rows, int64_t seq_len, int64_t d_model, int64_t heads, int64_t ffn_dim);
+// Whether norm1 and the projection in one launch are faster than in two.
+bool narrow_qkv_faster(int64_t rows, int64_t seq_len, int64_t d_model);
 hipError_t narrow_qkv_bf16(const bf16_t* x, const bf16_t* gamma, const bf16_t* beta, const bf16_t* w,
                            const bf16_t* bias, bf16_t* q, bf16_t* k, bf16_t* v_t, int64_t batch, int64_t seq_len,
                            int64_t d_model, int64_t heads, float eps, int cus, hipStream_t stream);

@@ -620,6 +620,13 @@ __global__ void __launch_bounds__(kWaves * kWave, 4) narrow_forward_kernel(const
   }
 }
 
+// Sequences of a workgroup: as many as its wavefronts (16 tokens each) and its
+// four 32-key blocks hold.
+int64_t sequences_per_group(int64_t S) {
+  const int64_t by_waves = kWaves / ((S + 15) / 16), by_keys = 4 / ((S + 31) / 32);
+  return by_waves < by_keys ? by_waves : by_keys;
+}
+
 template <int D, int HD>
 hipError_t launch(const NarrowArgs& a, hipStream_t st) {
   auto kernel = narrow_forward_kernel<D, HD>;
@@ -630,9 +637,8 @@ hipError_t launch(const NarrowArgs& a, hipStream_t st) {
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (attr != hipSuccess) return attr;
   }
-  const int nw = (a.S + 15) / 16, nk = (a.S + 31) / 32;
-  const int per_group = kWaves / nw < 4 / nk ? kWaves / nw : 4 / nk;
-  const int64_t groups = (static_cast<int64_t>(a.B) + per_group - 1) / per_group;
+  const int64_t per_group = sequences_per_group(a.S);
+  const int64_t groups = (a.B + per_group - 1) / per_group;
   hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups)), dim3(kWaves * kWave), kLds, st, a);
   return hipGetLastError();
 }
@@ -646,24 +652,34 @@ bool narrow_forward_supported(int64_t S, int64_t D, int64_t H, int64_t F) {
 }
 
 // Where one launch beats three launches a layer (narrow_rows.hip), measured on
-// MI355X, two layers, us (three a layer / one).  The sequence's time hardly moves
-// up to 8192 tokens (below 50 the host's launches count, not the kernels); one
-// launch's hardly moves up to 256 workgroups, and grows with the heads, which a
-// wavefront takes one after the other:
-//   d_model 32 and 64, 32 channels a head and more: always (d 64, hd 32, 8 x 128
-//     tokens level, 64 x 128 44.6 / 32.0, 256 x 128 65.5 / 34.0);
-//   d 128, hd 64 and 128: 32 x 128 56.3 / 58.1, 55.8 / 61.1, 64 x 128 55.2 /
-//     51.7, 57.7 / 55.3, 256 x 32 58.0 / 46.5;
-//   d 128, hd 32: 64 x 128 57.1 / 66.0, 128 x 128 81.9 / 68.3, 128 x 32 55.7 /
-//     59.5, 256 x 32 65.0 / 53.6;
-//   hd 8 at d 32: 32 x 128 level, 64 x 128 44.4 / 37.9; at d 64: 128 x 128 60.8 /
-//     71.0, 256 x 128 93.4 / 74.4, 256 x 32 68.5 / 45.3; at d 128: 128 x 128 109 /
-//     144, 256 x 128 155 / 156, 128 x 32 76.1 / 103, 256 x 32 112 / 96.8.
+// MI355X over 1 to 128 tokens a sequence and 1 to 16384 sequences, two layers,
+// us (three a layer / one).  The launches' time hardly moves up to a few
+// thousand tokens and then grows with the attention's workgroups, one per
+// sequence and head even where a sequence is a token; one launch's hardly moves
+// up to 256 workgroups of at most four sequences, and grows with the heads, which
+// a wavefront takes one after the other, and with the 16-token blocks of keys:
+//   d_model 32 and 64, 32 channels a head and more: always (d 64, hd 32: 8 x 128
+//     27.6 / 28.4, 128 x 64 37.5 / 25.3, 65536 x 1 2248 / 762);
+//   hd 8 at d 32: 32 x 128 29.2 / 34.8, 128 x 64 34.8 / 27.7; at d 64: 96 x 16
+//     34.0 / 35.1, 160 x 16 43.6 / 35.1, 160 x 65 60.9 / 55.9; at d 128: 128 x 64
+//     75.6 / 114, 192 x 24 89.5 / 91.7, 512 x 16 173 / 80.6, 65536 x 1 16561 / 3363;
+//   d 128, hd 32: 192 x 4 38.9 / 44.4, 240 x 12 47.1 / 45.2, 160 x 24 43.3 / 48.9,
+//     192 x 32 54.0 / 49.7, 96 x 64 48.5 / 54.8, 160 x 64 64.6 / 54.7, 64 x 128 53.2
+//     / 62.1, 96 x 128 71.6 / 62.3;
+//   d 128, hd 64: 128 x 4 35.2 / 38.2, 64 x 64 38.1 / 44.7, 128 x 64 52.5 / 45.3;
+//   d 128, hd 128, one workgroup per CU: 320 x 2 40.8 / 44.2, 64 x 64 37.3 / 49.0,
+//     256 x 32 60.1 / 48.0; many rounds of workgroups that are mostly padding, or
+//     whose wavefronts all have 128 keys, lose: 2048 x 1 98 / 88, 16384 x 1 567 /
+//     678, 512 x 128 120 / 107, 1024 x 128 194 / 214.
 bool narrow_forward_faster(int64_t B, int64_t S, int64_t D, int64_t H) {
   const int64_t hd = D / H;
-  if (hd == 8) return D == 32 ? B >= 32 || S <= 64 : B >= (D == 64 ? 176 : 240);
+  if (hd == 8) return D == 32 ? B >= 48 || S <= 64 : B >= (D == 128 ? 240 : S <= 16 ? 112 : 160);
   if (D < 128) return true;
-  return B >= (hd == 32 ? 96 : 48);
+  if (hd == 32) return B >= (S <= 16 ? 240 : S <= 32 ? 192 : S <= 64 ? 144 : 80);
+  if (hd == 64) return B >= (S <= 4 ? 160 : S <= 64 ? 80 : 56);
+  const int64_t groups = (B + sequences_per_group(S) - 1) / sequences_per_group(S);
+  if (S <= 8) return B >= (S <= 2 ? 320 : 240) && groups <= 1024;
+  return S <= 64 ? B >= 96 : B >= 64 && groups <= 768;
 }
 
 hipError_t narrow_forward_bf16(const NarrowForward& f, hipStream_t st) {

@@ -361,6 +361,16 @@ bool narrow_rows_supported(int64_t rows, int64_t seq_len, int64_t d_model, int64
          rows < (int64_t(1) << 31) - (int64_t(1) << 20) && seq_len <= (int64_t(1) << 23);
 }
 
+// The kernel pads every sequence to 16 tokens.  Even for one token that costs
+// less than the LayerNorm launch it saves, except at d_model 128, whose products
+// take twice d 64's time a slab, past about a thousand tokens (two layers, us,
+// this / the two launches: d 128 1024 x 1 65.4 / 62.0, 65536 x 1 2116 / 2001,
+// 16384 x 2 573 / 561, 16384 x 3 588 / 587, 64 x 1 37.0 / 41.2; d 64 1024 x 1 43.8 /
+// 54.7, 8192 x 1 186 / 189).
+bool narrow_qkv_faster(int64_t rows, int64_t seq_len, int64_t d_model) {
+  return d_model < 128 || seq_len > 2 || rows < 1024;
+}
+
 hipError_t narrow_qkv_bf16(const bf16_t* x, const bf16_t* gamma, const bf16_t* beta, const bf16_t* w,
                            const bf16_t* bias, bf16_t* q, bf16_t* k, bf16_t* v_t, int64_t batch, int64_t seq_len,
                            int64_t d_model, int64_t heads, float eps, int cus, hipStream_t st) {
