@@ -243,7 +243,7 @@ int run_encoder_forward(const void* x, void* out, void* workspace, const Encoder
   const bool no_split = !enc::gemm_has_split_tail(T, D, D, cus) && !enc::gemm_has_split_tail(T, F, D, cus) &&
                         !enc::gemm_has_split_tail(T, D, F, cus);
   bool one_launch = exact && num_layers > 0 && enc::narrow_forward_supported(seq_len, D, H, F) &&
-                    enc::narrow_forward_faster(batch, seq_len, D, H) && no_split &&
+                    enc::narrow_forward_faster(batch, seq_len, D, H, F) && no_split &&
                     (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
   for (int64_t i = 0; one_launch && i < 12 * num_layers + 2; ++i)
     one_launch = reinterpret_cast<uintptr_t>(weights[i]) % 16 == 0;

@@ -173,7 +173,7 @@ struct NarrowForward {
 };
 bool narrow_forward_supported(int64_t S, int64_t D, int64_t H, int64_t F);
 // Whether that launch is the faster one for a supported shape.
-bool narrow_forward_faster(int64_t B, int64_t S, int64_t D, int64_t H);
+bool narrow_forward_faster(int64_t B, int64_t S, int64_t D, int64_t H, int64_t F);
 hipError_t narrow_forward_bf16(const NarrowForward& f, hipStream_t stream);
 
 // Device addresses of the current device's GELU table (65536 bf16) and its

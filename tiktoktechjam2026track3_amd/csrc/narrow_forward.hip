@@ -652,12 +652,13 @@ bool narrow_forward_supported(int64_t S, int64_t D, int64_t H, int64_t F) {
 }
 
 // Where one launch beats three launches a layer (narrow_rows.hip), measured on
-// MI355X over 1 to 128 tokens a sequence and 1 to 16384 sequences, two layers,
-// us (three a layer / one).  The launches' time hardly moves up to a few
-// thousand tokens and then grows with the attention's workgroups, one per
-// sequence and head even where a sequence is a token; one launch's hardly moves
-// up to 256 workgroups of at most four sequences, and grows with the heads, which
-// a wavefront takes one after the other, and with the 16-token blocks of keys:
+// MI355X over 1 to 128 tokens a sequence and 1 to 20000 sequences, two layers, ffn
+// 128, us (three a layer / one; batch x tokens).  The launches' time hardly moves
+// up to a few thousand tokens and then grows with the attention's workgroups, one
+// per sequence and head even where a sequence is a token, ragged tiles costing more
+// than whole ones; one launch's hardly moves up to 256 workgroups of at most four
+// sequences, and grows with the heads, which a wavefront takes one after the other,
+// with the 32-key blocks and with ffn_dim (2 a layer less at 64, 3 at 32):
 //   d_model 32 and 64, 32 channels a head and more: always (d 64, hd 32: 8 x 128
 //     27.6 / 28.4, 128 x 64 37.5 / 25.3, 65536 x 1 2248 / 762);
 //   hd 8 at d 32: 32 x 128 29.2 / 34.8, 128 x 64 34.8 / 27.7; at d 64: 96 x 16
@@ -666,20 +667,27 @@ bool narrow_forward_supported(int64_t S, int64_t D, int64_t H, int64_t F) {
 //   d 128, hd 32: 192 x 4 38.9 / 44.4, 240 x 12 47.1 / 45.2, 160 x 24 43.3 / 48.9,
 //     192 x 32 54.0 / 49.7, 96 x 64 48.5 / 54.8, 160 x 64 64.6 / 54.7, 64 x 128 53.2
 //     / 62.1, 96 x 128 71.6 / 62.3;
-//   d 128, hd 64: 128 x 4 35.2 / 38.2, 64 x 64 38.1 / 44.7, 128 x 64 52.5 / 45.3;
-//   d 128, hd 128, one workgroup per CU: 320 x 2 40.8 / 44.2, 64 x 64 37.3 / 49.0,
-//     256 x 32 60.1 / 48.0; many rounds of workgroups that are mostly padding, or
-//     whose wavefronts all have 128 keys, lose: 2048 x 1 98 / 88, 16384 x 1 567 /
-//     678, 512 x 128 120 / 107, 1024 x 128 194 / 214.
-bool narrow_forward_faster(int64_t B, int64_t S, int64_t D, int64_t H) {
+//   d 128, hd 64: 128 x 12 36.9 / 38.6, 64 x 40 40.3 / 42.7, 128 x 40 52.4 / 42.8,
+//     64 x 64 38.1 / 44.7, 96 x 64 49.8 / 44.7; ffn 32 102 x 33 43.7 / 36.8;
+//   d 128, hd 128, one workgroup per CU: 320 x 2 40.8 / 44.2, 96 x 40 48.0 / 47.8,
+//     128 x 40 57.0 / 48.3, 64 x 64 37.3 / 49.0, 128 x 64 48.4 / 49.5; in many
+//     rounds of workgroups that are mostly padding, or whose wavefronts all have
+//     128 keys, 1321 x 1 71 / 78, 2048 x 1 98 / 88, 16384 x 1 567 / 678, 512 x 128
+//     120 / 107, 1024 x 128 194 / 214; ffn 64 2629 x 4 142 / 117.
+bool narrow_forward_faster(int64_t B, int64_t S, int64_t D, int64_t H, int64_t F) {
   const int64_t hd = D / H;
   if (hd == 8) return D == 32 ? B >= 48 || S <= 64 : B >= (D == 128 ? 240 : S <= 16 ? 112 : 160);
   if (D < 128) return true;
-  if (hd == 32) return B >= (S <= 16 ? 240 : S <= 32 ? 192 : S <= 64 ? 144 : 80);
-  if (hd == 64) return B >= (S <= 4 ? 160 : S <= 64 ? 80 : 56);
+  if (hd == 32) return B >= (S <= 16 ? 100 + F : S <= 32 ? 150 + F / 3 : S <= 64 ? 120 + F / 5 : 70 + F / 7);
+  const bool whole = S % 64 == 0;
+  if (hd == 64) return S <= 16 ? B >= 64 + 3 * F / 4 : B * S >= (whole ? 3800 + 12 * F : S <= 64 ? 34 * F : 4100);
   const int64_t groups = (B + sequences_per_group(S) - 1) / sequences_per_group(S);
-  if (S <= 8) return B >= (S <= 2 ? 320 : 240) && groups <= 1024;
-  return S <= 64 ? B >= 96 : B >= 64 && groups <= 768;
+  // (up to eight tokens: 36 us and 1/16 of ffn_dim a round of 256 workgroups,
+  // against 36 and 0.033 to 0.04 a sequence)
+  if (S <= 8)
+    return B >= (S <= 2 ? 224 : 112) + F && (36 + F / 16) * ((groups + 255) / 256) <= 36 + B * (32 + S) / 1000;
+  if (S <= 16) return B >= F;
+  return B * S >= (whole ? 5000 + 13 * F : S <= 64 ? 32 * F : 4100) && (S <= 64 || groups <= 768);
 }
 
 hipError_t narrow_forward_bf16(const NarrowForward& f, hipStream_t st) {
