@@ -151,22 +151,27 @@ def test_encoder_parity_narrow_one_launch(device, cfg, masking):
     "cfg",
     [TransformerConfig(64, 129, 128, 4, 128, 2, True), TransformerConfig(33, 259, 64, 1, 32, 2, False),
      TransformerConfig(9, 1001, 128, 1, 64, 1, True), TransformerConfig(300, 131, 32, 1, 128, 3, True),
-     TransformerConfig(8200, 1, 128, 16, 128, 1, False), TransformerConfig(100, 100, 128, 16, 32, 2, True),
+     TransformerConfig(200, 1, 128, 16, 128, 1, False), TransformerConfig(100, 100, 128, 16, 32, 2, True),
      TransformerConfig(31, 272, 64, 2, 64, 1, True), TransformerConfig(1, 16, 128, 16, 32, 2, True),
      TransformerConfig(2, 133, 128, 1, 128, 2, False), TransformerConfig(5, 129, 64, 8, 128, 1, True),
-     TransformerConfig(3, 700, 32, 1, 32, 2, True), TransformerConfig(8, 1000, 128, 2, 64, 2, True)],
+     TransformerConfig(3, 700, 32, 1, 32, 2, True), TransformerConfig(8, 1000, 128, 2, 64, 2, True),
+     TransformerConfig(70, 129, 32, 4, 32, 1, True), TransformerConfig(64, 130, 32, 1, 64, 2, False),
+     TransformerConfig(90, 137, 64, 2, 128, 1, False), TransformerConfig(5000, 3, 128, 1, 64, 1, True),
+     TransformerConfig(16385, 1, 128, 1, 128, 2, False), TransformerConfig(4200, 2, 128, 1, 32, 1, True)],
     ids=lambda c: f"{c.batch_size}x{c.seq_len}-d{c.d_model}-h{c.num_heads}-f{c.ffn_dim}-l{c.num_layers}",
 )
 @pytest.mark.parametrize("masking", ["none", "prefix", "general"])
 def test_encoder_parity_narrow_rows(device, cfg, masking):
-    """Narrow models that one launch does not serve: norm1 + QKV (its feature
-    blocks split among workgroups where the tokens are few) and the block tail
-    (with the final norm in the last one; past 8192 tokens by 16 tokens a
-    wavefront) around the attention.  Sequences that end inside a
-    16-token slab and inside V^T's 8-token padding, workgroups of 4, 8 and 16
-    wavefronts, every width; the oracle's bits (head dim 32 past 128 tokens:
-    the gate of the other parity tests, its P.V product reduces K in another
-    order at some lengths)."""
+    """Narrow models that one launch does not serve (sequences of more than 128
+    tokens, few of them, or very many short ones at head dim 128): norm1 + QKV
+    (its feature blocks split among workgroups where the tokens are few; from a
+    thousand sequences of one or two tokens on as two launches) and the block
+    tail (with the final norm in the last one; past 8192 tokens by 16 tokens a
+    wavefront, here at every width) around the attention.  Sequences that end
+    inside a 16-token slab and inside V^T's 8-token padding, sequences of one
+    token, workgroups of 4, 8 and 16 wavefronts; the oracle's bits (head dims 8
+    and 32 past 128 tokens: the gate of the other parity tests, their P.V product
+    reduces K in another order at some lengths)."""
     sd, candidate = build_models(cfg, 56, device)
     with torch.inference_mode():
         x, mask = generate_random_case(cfg, device, torch.bfloat16, 4, 0.6 if masking == "prefix" else 0.0, 1.0)
@@ -185,6 +190,102 @@ def test_encoder_parity_narrow_rows(device, cfg, masking):
         else:
             result = compare(ref, out, RTOL, ATOL)
             assert result["passed"], result
+
+
+@pytest.mark.parametrize("batch,seq_len", [(300, 1), (9000, 1), (2, 16), (70, 130)])
+@pytest.mark.parametrize("d_model", [64, 128])
+def test_narrow_rows_around_the_online_attention(device, d_model, batch, seq_len):
+    """The one-pass attention (head dim 64) between the narrow launches, at any
+    sequence length: bit for bit the separate launches, which a weight that is
+    not 16-byte aligned selects; with one key a query, whose weight is 1, the
+    oracle's bits too."""
+    cfg = TransformerConfig(batch, seq_len, d_model, d_model // 64, 128, 2, True)
+    sd, candidate = build_models(cfg, 59, device)
+    with torch.inference_mode():
+        x, mask = generate_random_case(cfg, device, torch.bfloat16, 6, 0.4, 1.0)
+        kv_len, row_mask = native.mask_lengths(mask), mask.contiguous().view(torch.uint8)
+        table, eps, _ = candidate._native_weights(device, 0)
+        shifted = torch.empty(d_model + 4, device=device, dtype=torch.bfloat16)[4:]
+        shifted.copy_(candidate.final_norm.bias)
+        assert shifted.data_ptr() % 16 == 8
+        other = table.clone()
+        other[-1] = shifted.data_ptr()
+        outs = []
+        for weights in (table, other):
+            out = torch.full_like(x, float("nan"))
+            native.encoder_forward(x, out, candidate._native_workspace(x), weights, cfg.num_heads, cfg.ffn_dim,
+                                   cfg.num_layers, eps, cfg.causal, kv_len, None, row_mask, online_attention=True)
+            outs.append(out)
+        assert torch.equal(*outs)
+        if seq_len == 1:
+            assert torch.equal(outs[0], encoder_forward(sd, x, mask, cfg.causal, cfg.num_heads, cfg.num_layers))
+
+
+# Patterns at the edges of the compact table's two slices, zeros, subnormals,
+# the largest finite values and some between, each sign.
+GELU_EDGES = [s | a for s in (0, 0x8000) for a in
+              [0, 1, 0x7F, 0x80, 0x3880, 0x397D, 0x397E, 0x397F, 0x3980, 0x3981, 0x3982, 0x40AF, 0x40B0, 0x40B1,
+               0x40B2, 0x40B3, 0x4100, 0x7F7E, 0x7F7F] + list(range(0x3985, 0x40AF, 42))]
+
+
+@pytest.mark.parametrize(
+    "cfg",
+    [TransformerConfig(200, 32, 128, 4, 128, 1, True), TransformerConfig(64, 33, 64, 2, 128, 1, False),
+     TransformerConfig(30, 128, 32, 1, 32, 1, True), TransformerConfig(64, 130, 128, 4, 128, 1, True),
+     TransformerConfig(65, 129, 64, 1, 64, 1, False)],
+    ids=["one-launch-d128", "one-launch-d64", "one-launch-d32", "tail-d128", "tail-d64"],
+)
+def test_narrow_gelu(device, cfg):
+    """The narrow kernels' GELU at and past the edges of its table, from the
+    table and (ready flag cleared) from the erf, and the table read at all (one
+    planted entry).  With out_proj and ffn_in's weights zero, ffn_out a unit
+    matrix and a zero input, the block's output is the GELU of ffn_in's bias."""
+    d, f = cfg.d_model, cfg.ffn_dim
+    _, candidate = build_models(cfg, 58, device)
+    layer = candidate.layers[0]
+    x = torch.zeros(cfg.batch_size, cfg.seq_len, d, device=device, dtype=torch.bfloat16)
+    workspace = candidate._native_workspace(x)
+
+    def block(patterns):
+        bits = torch.zeros(f, device=device, dtype=torch.int32)
+        bits[: len(patterns)] = torch.tensor(patterns, device=device, dtype=torch.int32)
+        layer.ffn_in.bias.copy_(bits.to(torch.int16).view(torch.bfloat16))
+        table, eps, packed = candidate._native_weights(device, 0)
+        out = torch.empty_like(x)
+        native.encoder_forward(x, out, workspace, table, cfg.num_heads, f, 1, eps, cfg.causal, None, None, None,
+                               final_norm=False, packed_weights=packed)
+        hidden = torch.nn.functional.gelu(layer.ffn_in.bias).expand(64, f)
+        return out, torch.nn.functional.linear(hidden, layer.ffn_out.weight)[0]
+
+    per_call = min(d, f)
+    planted = 0x3F80  # 1.0
+    with torch.no_grad():
+        for p in (layer.attention.out_proj.weight, layer.attention.out_proj.bias, layer.ffn_in.weight,
+                  layer.ffn_out.weight, layer.ffn_out.bias):
+            p.zero_()
+        layer.ffn_out.weight[:per_call, :per_call] = torch.eye(per_call, device=device)
+        block([0])  # the table is filled
+        try:
+            for ready in (1, 0):
+                native.debug_gelu_table(device, ready=ready)
+                for at in range(0, len(GELU_EDGES), per_call):
+                    out, ref = block(GELU_EDGES[at:at + per_call])
+                    assert torch.equal(out[..., :per_call], ref[:per_call].expand_as(out[..., :per_call])), (ready, at)
+                # a value that is not finite reaches every feature of ffn_out
+                layer.ffn_out.weight[:, 0] = 1
+                for pattern in (0x7F80, 0xFF80, 0x7FC0, 0xFFC0, 0x7F81):
+                    out, ref = block([pattern])
+                    same = out == ref[0] if pattern == 0x7F80 else torch.isnan(out) & torch.isnan(ref[0])
+                    assert bool(same.all()), (ready, hex(pattern))
+                layer.ffn_out.weight[1:, 0] = 0
+            native.debug_gelu_table(device, ready=1, entry=planted, value=0x4120)
+            out, _ = block([planted, 0x3F81])
+            assert bool((out[..., 0] == 10.0).all()), "the table is read"
+            native.debug_gelu_table(device, ready=0)
+            out, ref = block([planted, 0x3F81])
+            assert torch.equal(out[..., :2], ref[:2].expand_as(out[..., :2])), "the erf ignores the table"
+        finally:
+            native.debug_gelu_table(device, ready=1, entry=planted, value=-1)
 
 
 @pytest.mark.parametrize("seq_len", [17, 29, 99])

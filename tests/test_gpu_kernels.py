@@ -255,18 +255,19 @@ def test_linear_narrow_and_d128_shapes_bitwise(device, m, n, k):
     assert torch.equal(out[mask], (res + ref)[mask]) and torch.equal(out[~mask], res[~mask])
 
 
-@pytest.mark.parametrize("packed", [False, True], ids=["plain", "packed"])
+RING_TILES = [(257, 64, 64), (300, 192, 192), (1000, 1024, 1024), (512, 1088, 128), (2048, 1024, 64),  # 64 x 64 tiles
+              (777, 4096, 256), (1025, 2176, 512), (1500, 4096, 512), (1537, 4096, 192), (2331, 2048, 512),  # past them
+              (9057, 1536, 2048), (2048, 2048, 4096)]  # (GELU by rounds: 256 x 256 and 256 x 128)
+
+
 @pytest.mark.parametrize(
-    "m,n,k",
-    [(257, 64, 64), (300, 192, 192), (1000, 1024, 1024), (512, 1088, 128), (2048, 1024, 64),  # 64 x 64 tiles
-     (777, 4096, 256), (1025, 2176, 512), (1500, 4096, 512), (1537, 4096, 192), (2331, 2048, 512)],  # past them
+    "m,n,k,packed",
+    [(*shape, packed) for packed in (False, True) for shape in RING_TILES if not packed or native.prepack_rows(*shape[1:])],
 )
 def test_linear_ring_tiles_bitwise(device, m, n, k, packed):
     """The ring kernel's smaller tiles (64 x 64 up to two per CU, then 128 x
-    128 with one or two per CU and 256 x 128): one K block and more, ragged
-    last rows, every epilogue, both weight layouts, bit for bit torch."""
-    if packed and native.prepack_rows(n, k) == 0:
-        pytest.skip("no packed form")
+    128 with one or two per CU, 256 x 128 and 256 x 256): one K block and more,
+    ragged last rows, every epilogue, both weight layouts, bit for bit torch."""
     a, w, bias, res, _ = _linear_case(device, m, n, k, 31 * m + n + k)
     wp = native.prepack_weight(w) if packed else None
     ref = F.linear(a, w, bias)
@@ -738,12 +739,14 @@ def test_attention_head_dims_bitwise(device, hd, b, h, s, causal, prefix, exact)
     [(32, 172, 1, 257, True, "none", 1.0), (32, 64, 4, 777, False, "prefix", 1.0), (32, 32, 4, 500, True, "bytes", 8.0),
      (32, 4, 8, 2048, True, "none", 1.0), (8, 32, 8, 320, True, "prefix", 1.0), (8, 16, 4, 1000, False, "bytes", 1.0),
      (256, 1, 1, 129, True, "none", 1.0), (256, 2, 3, 777, False, "prefix", 4.0), (256, 1, 2, 2048, True, "bytes", 1.0),
-     (256, 64, 4, 257, True, "none", 1.0), (256, 40, 4, 500, False, "bytes", 1.0)],
+     (256, 64, 4, 257, True, "none", 1.0), (256, 40, 4, 500, False, "bytes", 1.0),
+     (32, 90, 4, 300, False, "none", 1.0), (32, 40, 4, 800, True, "none", 1.0), (32, 100, 4, 500, True, "prefix", 1.0),
+     (8, 120, 4, 300, True, "bytes", 4.0), (8, 40, 4, 800, True, "none", 1.0), (8, 64, 4, 500, True, "prefix", 1.0)],
 )
 def test_attention_streamed_rows_other_head_dims(device, hd, b, h, s, causal, mask_kind, q_gain):
-    """Streamed rows (head dims 8 and 32 past 256 keys in grids that fill the
-    chip: four wavefronts per SIMD, half-tile sweeps; head dim 256 past 128
-    keys: four wavefronts per 128 queries in grids of any size), at one key
+    """Streamed rows (head dims 8 and 32 past 256 keys, with four wavefronts per
+    SIMD and half-tile sweeps or with two, on both sides of the rule; head dim
+    256 past 128 keys: four wavefronts per 128 queries in grids of any size), at one key
     past the resident rows, ragged last tiles, the longest rows, each mask and
     the IEEE division path (q_gain).  Head dim 256 and power-of-32 lengths give
     the oracle's bits; for head dims 8 and 32 the reference's P.V product
