@@ -562,6 +562,24 @@ def test_packed_copies_follow_in_place_weight_updates(device, graph):
     assert torch.equal(after, plain)
 
 
+def test_narrow_models_make_no_packed_copies(device):
+    """Narrow models read the plain weights: no packed copies at any number of
+    rows, and the graph, whose kernels read the weights in place, follows an
+    in-place update without a new capture."""
+    cfg = TransformerConfig(16, 128, 128, 4, 128, 2, True)  # 2048 rows, graph-eligible
+    _, candidate = build_models(cfg, 13, device)
+    g = torch.Generator(device=device).manual_seed(3)
+    with torch.inference_mode():
+        x = torch.randn(16, 128, 128, generator=g, device=device).bfloat16()
+        before = candidate(x)
+        assert candidate._hip.packed is None and not candidate._pack_enabled(1 << 20)
+        candidate.layers[1].ffn_in.weight.mul_(0.5)
+        after = candidate(x)
+        assert candidate._cuda_graph_capture_count == 1
+        assert torch.equal(after, candidate._forward_native(x, None, "all_true"))
+    assert not torch.equal(before, after)
+
+
 def test_online_attention_encoder_stays_close(device):
     """The opt-in one-pass attention: its bf16 weight-rounding noise compounds
     over the layers, so it is held to a looser bound than the reference's gate

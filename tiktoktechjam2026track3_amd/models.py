@@ -69,9 +69,11 @@ def even_row_block(seq_len: int, limit: int) -> int:
 
 # Token count up to which the candidate captures a HIP graph (launch-bound shapes).
 GRAPH_MAX_TOKENS = 4096
-# The tile-packed weight copies are read only by the wide GEMM kernel's larger
-# tiles; inputs of fewer rows than this leave them unmade.
+# The tile-packed weight copies are read by the ring GEMM kernel, from 257 rows
+# on.  They pay on its larger tiles; inputs of fewer rows than this leave them
+# unmade, as do narrow models, whose launches read the plain weights.
 PACK_MIN_ROWS = 1024
+NARROW_MAX_WIDTH = 128
 
 
 class UnsupportedShapeError(NotImplementedError):
@@ -539,6 +541,8 @@ class UserOptimizedTransformer(BaselineTransformer):
 
         cfg = self.config
         d, f = cfg.d_model, cfg.ffn_dim
+        if max(d, f) <= NARROW_MAX_WIDTH:
+            return False
         return rows >= PACK_MIN_ROWS and cfg.num_layers > 0 and all(
             native.prepack_rows(n, k) for n, k in ((3 * d, d), (d, d), (f, d), (d, f)))
 
