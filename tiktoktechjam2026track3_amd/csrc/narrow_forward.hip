@@ -278,11 +278,13 @@ __device__ __forceinline__ void block_product(const bf16_t* frags, int lane, con
 }
 
 // What bounds it: VALU issue (rocprofv3 on 10000 sequences of 128 tokens, d_model
-// 128, head dim 32: 80% of the cycles, about 4700 instructions a wavefront and
-// layer, more than half of them the exact softmax); in a small batch the
-// latency of one workgroup, 30 us a layer at 32 channels a head.  16 tokens a
-// wavefront leave 128 registers, four wavefronts per SIMD (two workgroups of 77
-// KiB per CU; one at head dim 128): 32 tokens a wavefront at two per SIMD ran
+// 128, head dim 32: 79% of the cycles at four an instruction, 4857 instructions a
+// wavefront and layer with 236 MFMAs, more than half of them the exact softmax);
+// in a small batch the latency of one workgroup, 30 us a layer at 32 channels a
+// head.  16 tokens a wavefront leave 128 registers, four wavefronts per SIMD (two
+// workgroups of 77 KiB per CU; one at head dim 128), at the price of spills: 7 to
+// 57 vector registers at d_model 128 and at head dim 8 of 64, 18 to 54 scalar
+// ones, to vector lanes, everywhere.  32 tokens a wavefront at two per SIMD ran
 // the four layers of that batch in 3.71 ms against 3.17 ms here, the launches
 // this replaced (norm, QKV, attention, out_proj, norm, ffn_in, ffn_out a layer)
 // in 7.30 ms.
