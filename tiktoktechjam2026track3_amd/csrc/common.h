@@ -124,6 +124,15 @@ __device__ __forceinline__ float gelu_erf(float x) {
   return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));
 }
 
+// The GELU of a bf16 value from a table: torch's GELU of every bf16 pattern
+// (checked exhaustively) needs one only for the magnitudes a = bits & 0x7fff in
+// [kGeluLo, kGeluHi] (|x| from 2.4e-4 to 5.53).  Outside it follows from x:
+//   a < kGeluLo:  bf16(0.5 x)  (erf(x / sqrt 2) is below half an ulp of 1);
+//   a > kGeluHi:  x for x > 0, -0 for x < 0, the canonical NaN 0x7fc0 for
+//                 NaN inputs and for -inf (-inf * 0).
+constexpr uint32_t kGeluLo = 0x3980u;
+constexpr uint32_t kGeluHi = 0x40b1u;
+
 // s_waitcnt immediate (gfx9 encoding): wait until at most `vm` vector-memory
 // and `lgkm` LDS operations of this wavefront are outstanding.
 constexpr int waitcnt_imm(int vm, int lgkm) {

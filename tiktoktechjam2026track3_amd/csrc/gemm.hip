@@ -95,19 +95,12 @@ __global__ void gelu_entry_set_kernel(uint32_t x, int32_t value) {
 }
 
 // The wide kernel's GELU epilogue reads a compact copy of the table from LDS:
-// for each sign, the bf16 magnitudes a = bits & 0x7fff in [kGeluLo, kGeluHi]
-// (|x| from 2.4e-4 to 5.53; 7.2 KiB for both signs, which leaves two 256x128
-// workgroups per CU room).  Outside that range the values follow from x
-// itself, as torch's GELU of every bf16 pattern shows (checked exhaustively):
-//   a < kGeluLo:  bf16(0.5 x)  (erf(x / sqrt 2) is below half an ulp of 1);
-//   a > kGeluHi:  x for x > 0, -0 for x < 0, the canonical NaN 0x7fc0 for
-//                 NaN inputs and for -inf (-inf * 0).
-// The table region is filled from g_gelu_table's two slices (the entries for
-// a positive x are x itself from 2.77 on).  A pass whose eight values all lie
-// in the range (nearly every pass for activations of unit scale) does only the
-// lookups; otherwise the pass evaluates the rules above per value.
-constexpr uint32_t kGeluLo = 0x3980u;
-constexpr uint32_t kGeluHi = 0x40b1u;
+// for each sign the magnitudes in [kGeluLo, kGeluHi] (common.h; 7.2 KiB for both,
+// which leaves two 256x128 workgroups per CU room), filled from g_gelu_table's two
+// slices (the entries for a positive x are x itself from 2.77 on).  A pass whose
+// eight values all lie in the range (nearly every pass for activations of unit
+// scale) does only the lookups; otherwise the pass evaluates common.h's rules per
+// value.
 constexpr int kGeluSpan = static_cast<int>(kGeluHi - kGeluLo + 1);  // entries per sign
 static_assert(kGeluSpan % 2 == 0 && kGeluLo % 2 == 0, "whole 4-byte words per slice");
 

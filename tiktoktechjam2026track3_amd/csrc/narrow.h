@@ -27,11 +27,8 @@
 namespace enc {
 namespace narrow {
 
-// The exact GELU's compact table (bf16 patterns of magnitude [kGeluLo,
-// kGeluHi], see gelu_compact in gemm.hip for the rules outside it): two slices
-// of 231 16-byte chunks, copied to LDS by the workgroup.
-constexpr uint32_t kGeluLo = 0x3980u;
-constexpr uint32_t kGeluHi = 0x40b1u;
+// The exact GELU's compact table: two slices of 231 16-byte chunks, copied to
+// LDS by the workgroup.
 constexpr int kGeluChunks = 231;                  // 16-byte chunks per sign, 1842 entries and 6 more
 constexpr int kGeluSliceBytes = kGeluChunks * 16;
 static_assert((kGeluHi - kGeluLo + 1) * 2 <= kGeluSliceBytes && (kGeluLo * 2) % 16 == 0, "table slices");
@@ -186,7 +183,9 @@ __device__ __forceinline__ void row_norm(const u32x4 (&x)[D / 32], const bf16_t*
 }
 
 // GELU of eight bf16 values: through the table in LDS (tab: two slices of
-// kGeluSliceBytes, magnitudes from kGeluLo) or, with no table, the erf.
+// kGeluSliceBytes, magnitudes from kGeluLo; common.h's rules outside it) or, with
+// no table, the erf.  (As gelu8_lds in gemm.hip; one function for both cost these
+// kernels, at the edge of their registers, 1 to 3% in small batches.)
 __device__ __forceinline__ u32x4 gelu8(u32x4 w, const char* tab, bool table) {
   if (table) {
     uint32_t u[8];
