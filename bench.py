@@ -5,7 +5,7 @@
 
 A step is one forward of ``UserOptimizedTransformer`` (the drop-in candidate
 of transformer_benchmark/models.py:922-1239) over one batch of synthetic input
-already resident in HBM.  The headline workload is BASELINE configuration c5
+already resident in HBM.  The headline workload is configuration c5
 (B=32, S=100000, D=1024, H=16, FFN=1024, L=2, bf16, non-causal, weights seeded
 with 4, timing input seeded with 4 + 100000 as in timing.py:123): the largest
 configuration, which fits one GPU only because scores are never materialised.
@@ -193,7 +193,7 @@ def copy_calibration(mib, torch):
 # ----------------------------------------------------------- CPU baseline ----
 
 def host_cpu():
-    """CPU model and logical core count of the host (the GPU box's, in a GPU run)."""
+    """CPU model and logical core count of the host the process runs on."""
     model = "unknown"
     try:
         for line in Path("/proc/cpuinfo").read_text().splitlines():

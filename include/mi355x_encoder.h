@@ -112,8 +112,8 @@ int enc_linear_order_clear(void);
 /* Test hook, no counterpart in the reference (for tests that must tell the
  * GELU epilogue's two paths apart; they give the same bits by design).  On
  * the current device, enqueued on stream after the GELU table's fill:
- * ready >= 0 sets the table's ready flag (0 makes every GELU epilogue of the
- * wide GEMM evaluate the erf, 1 lets it read the table); entry in [0, 65535]
+ * ready >= 0 sets the table's ready flag (0 makes every GELU of the wide GEMM
+ * and of the narrow models' kernels evaluate the erf, 1 lets it read the table); entry in [0, 65535]
  * overwrites that bf16 pattern's table entry with value in [0, 65535], or
  * recomputes it when value is -1.  Not for production use: a changed entry
  * changes the GELU of every later product until it is restored. */

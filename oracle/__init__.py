@@ -1,7 +1,7 @@
 """Test infrastructure only: the CPU restatement of the reference encoder forward.
 
 Only ``tests/``, ``__graft_entry__.smoke()`` and the ``cpu_baseline`` leg of
-``bench.py`` may import this package, and only as the checker (or the timed CPU
+``bench.py`` may import this package, and only as the oracle (or the timed CPU
 baseline).  The product (``tiktoktechjam2026track3_amd``) never imports it.
 """
 

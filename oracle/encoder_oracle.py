@@ -3,8 +3,8 @@
 A from-scratch, functional restatement of the reference Transformer encoder
 forward (transformer_benchmark/models.py of Sober7135/TikTokTechJam2026Track3)
 written over a plain ``state_dict``, plus the reference's seeded weight init and
-input generator.  It runs on whatever device its tensors live on: on the CPU
-here, and on torch-ROCm on the GPU box, where it is the checker the HIP path is
+input generator.  It runs on whatever device its tensors live on: on the
+CPU, and with torch-ROCm on the GPU, where it is the oracle the HIP path is
 compared against.  It is also the timed CPU baseline of ``bench.py``.
 
 Functions and the reference lines they restate:

@@ -75,7 +75,7 @@ def test_cli_remaining_official_cases_1_to_13_pass(tmp_path):
 
 def test_cli_encoder_config_c1_on_the_gpu_box(tmp_path):
     """c1 (B=2, S=128, D=256, H=4, FFN=1024, L=2, fp32, seed 0) is the
-    reference's CPU smoke case: on the GPU box the CLI still runs it through
+    reference's CPU smoke case: with a GPU present the CLI still runs it through
     the candidate's CPU path (the reference's CPU fallback contract) and holds
     it to the reference gate against the baseline, bit for bit."""
     out = tmp_path / "c1.json"

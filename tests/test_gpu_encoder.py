@@ -414,7 +414,7 @@ def _c5_sampled(device, causal: bool):
 
 
 def _summary(capsys, name, results):
-    """One line past pytest's output capture: the driver's log tail shows it."""
+    """One line past pytest's output capture, for the log's tail."""
     passed = sum(bool(r["passed"]) for _, r, _ in results)
     worst = max(r["max_abs_error"] for _, r, _ in results)
     bitwise = min(bw for _, _, bw in results)

@@ -16,7 +16,7 @@ from tiktoktechjam2026track3_amd import native
 
 pytestmark = pytest.mark.gpu
 
-RTOL = 1.6e-2  # the build's bf16 gate
+RTOL = 1.6e-2  # the bf16 gate: |d| < 1e-2 or |d| < 1.6e-2 |ref|
 ATOL = 1e-2
 
 

@@ -512,7 +512,7 @@ class UserOptimizedTransformer(BaselineTransformer):
         """The parameters of every layer, 12 each in the C ABI's order, then
         final_norm's two: the ones in place now.  Read from the modules' own
         dictionaries: every call walks them all, and attribute access on modules
-        made that most of its host time (four layers, MI355X box: a call of
+        made that most of its host time (four layers: a call of
         three launches a layer 115 -> 73 us, of one launch 85 -> 41 us)."""
         params: List[torch.Tensor] = []
         for layer in self._modules["layers"]._modules.values():

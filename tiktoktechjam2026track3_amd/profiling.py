@@ -26,7 +26,7 @@ with one; it is the largest ``__amd_rocclr_copyBuffer`` dispatch), so the
 traffic figures are in bytes of HBM actually moved.
 
     python -m tiktoktechjam2026track3_amd.profiling \\
-        --trace gpurun_out/trace_c2 --fetch gpurun_out/fetch_c2 --write gpurun_out/write_c2 \\
+        --trace prof/trace_c2 --fetch prof/fetch_c2 --write prof/write_c2 \\
         --copy-mib 256 --workload c2 --label ffn_out_residual='gemm_bf16_kernel<64, 64, 3' \\
         --command "..." --out profiles/encoder_c2.md --traffic profiles/traffic.json
 

@@ -15,7 +15,7 @@ that begins at s and ends with the -2^20, so per tile the smallest surviving
 block is s.  Which tiles split, and where, were checked bitwise against the
 library on random inputs (tests/test_gpu_kernels.py).
 
-Usage (on the GPU box):  python -m tiktoktechjam2026track3_amd.streamk_probe 3200000 100000
+Usage (needs the GPU):  python -m tiktoktechjam2026track3_amd.streamk_probe 3200000 100000
 prints the header to stdout, stamped with the device's CU count and the torch
 and HIP versions.  The probe is a maintainer tool: nothing at run time imports
 it.  At run time the plugin measures the order of every product shape it runs
