@@ -1841,17 +1841,17 @@ int pick_big_tile(int64_t M, int64_t N, int64_t K, const bf16_t* A, const bf16_t
   // 256x256, 256x128 and 128x128 tiles, and several rounds of 128x128 tiles
   // slow each other (9000x2048x2048: 5 rounds 88.8 us, 3 of 256x128 84.9).
   // (2331x2048x2048, where 128x128 tiles need a second round: 33.5 -> 25.5 us on
-  // 256x128; 1500x4096x1024 20.4 -> 17.3; QKV 2048x3072x1024 24.2 -> 20.8.)  0.85
-  // takes five rounds of 256x128 for three of 256x256 (us: 8501x4096x4096 258 / 280,
-  // 6000x6144x2048 158 / 165, 36065x1024x1024 level) but not seven for four
-  // (54903x1024x1024 121 / 117, 56177x1024x4096 433 / 397; with a K of 256 alone
-  // 53443x1024 48.6 / 51.3).
+  // 256x128; 1500x4096x1024 20.4 -> 17.3; QKV 2048x3072x1024 24.2 -> 20.8.)  0.83
+  // leaves three rounds of 256x256 in place of five of 256x128, level or slower
+  // alone (us: 6000x6144x2048 165 / 158, 8501x4096x4096 280 / 258) but faster inside a
+  // forward, whose operands are not in the caches yet (one layer of 9 x 2048 tokens
+  // at d_model 2048 2257 / 2356, 36 x 1000 at 1024 1243 / 1275).
   auto cost = [&](int bm, int bn, double eff) {
     const int64_t rounds = (tiles(bm, bn) + num_cus - 1) / num_cus;
     return static_cast<double>(rounds) * bm * bn / eff;
   };
   const double c256 = N % 256 == 0 ? cost(256, 256, 1.0) : 1e30;
-  const double c128 = cost(256, 128, 0.85), c64 = cost(128, 128, 0.68);
+  const double c128 = cost(256, 128, 0.83), c64 = cost(128, 128, 0.68);
   if (c256 <= c128 && c256 <= c64) return 256256;
   if (c128 > c64) return 128128;
   // V^T of sequences of one or two tokens is mostly padding, up to eight times
